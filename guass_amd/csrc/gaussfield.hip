@@ -222,14 +222,22 @@ FwdLayout fwd_layout(const Problem& p) {
 // per moment, on S different cache lines.
 // It must be zero before the first backward; every backward leaves it zero again
 // (k_bwd_finish clears what it reads), so a workspace kept across calls is zeroed once.
+constexpr int32_t kMaxStripes = 32;
 struct BwdLayout {
   size_t acc, total;
 };
+// The size is that of the largest need of any K up to this one (backward_stripes gives fewer
+// Gaussians more stripes: S * K <= blocks where it adds any), so that it grows with K and a
+// workspace sized for a K capacity holds every smaller K.
+int64_t tile_blocks16(const Problem& p) {
+  return (int64_t)p.R * p.C * (p.tile_out == 32 && p.tile_in == 32 ? 4 : 1);
+}
 BwdLayout bwd_layout(const Problem& p) {
   BwdLayout L;
   size_t o = sizeof(WsHeader);
   L.acc = o;
-  o = align256(o + sizeof(float) * 8 * (size_t)p.S * (size_t)p.K);
+  const int64_t slots = std::max<int64_t>((int64_t)p.S * p.K, std::min<int64_t>(kMaxStripes * p.K, tile_blocks16(p)));
+  o = align256(o + sizeof(float) * 8 * (size_t)slots);
   L.total = o;
   return L;
 }
@@ -3616,9 +3624,17 @@ __global__ __launch_bounds__(256) void k_selftest_softplus(unsigned long long* o
 // stripe lines depends on the accumulators' base address: above 16,384 tiles 16 stripes left
 // cfg5's reduction at 37-56 us over placements, 32 at 35-39 us (64: the finish cost more than it
 // saved).  Without hot Gaussians the stripes cost the finish 0.5-1.9 us.
-int32_t backward_stripes(int64_t K, int64_t T) {
-  (void)K;
-  return T >= 16384 ? 32 : (T >= 8192 ? 8 : (T >= 2048 ? 4 : 1));
+// Few Gaussians on many 16x16 blocks (wide Gaussians: a fresh adapter, or 32x32 tiles, whose four
+// waves add one by one) meet the same lines from every block: S then doubles, up to 32, while there
+// is no more than a slot per block, S * K <= blocks.  A 1280x1280 field of 256 wide Gaussians on 32x32 tiles (61
+// a tile) took its reduction from 100 us with one stripe to 40 with 8 and 35 with 32; a batch of 28
+// such layers from 526 to 366 us; 320x320 with K = 32 from 16.5 to 8.7 us.  With
+// more slots than blocks the finish loses what the reduction gains (28 trained layers of K = 1024:
+// 84.6 -> 81.9 us against 5.2 -> 7.5 us at 1.25 slots a block).
+int32_t backward_stripes(int64_t K, int64_t T, int64_t blocks) {
+  int32_t S = T >= 16384 ? 32 : (T >= 8192 ? 8 : (T >= 2048 ? 4 : 1));
+  while (K > 0 && S < kMaxStripes && 2 * S * K <= blocks) S *= 2;
+  return S;
 }
 
 int make_problem(const gf_field_config* cfg, int64_t M, int64_t N, int64_t K, Problem* p) {
@@ -3653,7 +3669,7 @@ int make_problem(const gf_field_config* cfg, int64_t M, int64_t N, int64_t K, Pr
     p->q_hi = INFINITY;
   }
   p->normalize = cfg->normalize ? 1 : 0;
-  p->S = backward_stripes(K, R * C);
+  p->S = backward_stripes(K, R * C, tile_blocks16(*p));
   p->mu_tanh = 0;
   p->mask_clamp = (cfg->has_clamp_quad && cfg->clamp_quad < 80.0) ? 1 : 0;
   p->heavy = 0;  // set per launch (heavy_threshold)
@@ -4839,6 +4855,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
     Problem pc;
     rc = make_problem(cfg, in.out_features, in.in_features, kc, &pc);
     if (rc) return set_err(rc, "layer %zu: k_capacity %lld invalid", i, (long long)kc);
+    ly.p.S = pc.S;  // the capacity's, which the finish grid is sized for
     if (t32 && !quad_render(ly.p))
       return set_err(GF_E_INVALID_ARGUMENT,
                      "layer %zu: batched 32x32 tiles need the mask path (1 <= k <= %lld, tile columns within LDS)",
