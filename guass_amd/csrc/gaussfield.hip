@@ -1595,6 +1595,219 @@ __device__ void order_segment_wave(int64_t* seg, int64_t n, int64_t K, int32_t* 
   }
 }
 
+// Lanes 0..31 of the result: a + (a of lane + 32); lanes 32..63: (b of lane - 32) + b
+// (v_permlane32_swap exchanges lanes 32..63 of its first operand with lanes 0..31 of its second).
+__device__ inline float swap32_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Rows of 16 lanes: row 2i + 0 of the result: a + (a of lane + 16); row 2i + 1: (b of lane - 16) + b
+// (v_permlane16_swap exchanges the odd rows of its first operand with the even rows of its second).
+__device__ inline float swap16_add(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+
+// ------------------------------------------------------------------------------------------
+// Wide Gaussians: one whose exponent changes little over a 16x16 block is a short polynomial there.
+// About the block's middle (X, Y), with xi = (x - X) / sx and eta = (y - Y) / sy (sx, sy powers of
+// two, |xi|, |eta| <= 1),
+//   e = e0 exp(-(L1 xi + L2 eta + Q11 xi^2 + Q12 xi eta + Q22 eta^2)) = sum_ab c_ab xi^a eta^b,
+//   (a + 1) c_{a+1,b} = -(L1 c_ab + 2 Q11 c_{a-1,b} + Q12 c_{a,b-1}),   c_00 = e0,
+// cut at total degree kPolyDeg.  The render sums the c_ab of a block's wide Gaussians (a lane each)
+// and evaluates one polynomial; the backward takes the block's moments of dL/d(delta-W) against
+// xi^a eta^b once and each Gaussian's six moments from its c_ab and those.  The work per (Gaussian,
+// block) is 45 coefficients of three FMAs instead of 256 exponentials.
+//
+// What the cut leaves out.  With l = max |L1 xi| + |L2 eta| and k the same bound of the quadratic terms, the terms past
+// degree D of exp(l t + k t^2) bound it (times e0, at a corner of the block): 1e-6 for D = 8 along l + 8 k = 0.85, and
+// growing like (l + 8 k)^(D + 1).  A Gaussian is wide in a block where e0 times that stays below 1e-6, that is where
+// l + 8 k <= kPolyReach e0^(-1 / 9).  A round Gaussian of 36 elements' sigma or more is wide in every block its 3-sigma
+// box meets.  The block's average is a twentieth of the corner's, and against 64 bits the polynomials are closer than
+// summing exponentials (Gaussians of 35-120 elements' sigma: 1.5e-7..2.2e-7 of the norm against 2.2e-7..3.1e-7):
+// 64 lanes' terms add in a tree, and one exponential's argument is rounded instead of 256.
+constexpr int kPolyDeg = 8;
+constexpr float kPolyReach = 0.85f;
+// Fewer wide Gaussians than this in 64 do not repay the reduction and the evaluation (about 450
+// instructions a block against 24-34 a Gaussian).
+constexpr int kPolyMin = 24;
+constexpr int kPolyMore = 8;  // and a further 64's, whose sums join the first's
+constexpr float kPolyMaxQ = 24.0f;     // (farther ones, whose reach would say little, go element by element)
+constexpr float kPolyMaxAmp = 1e30f;  // amplitudes past this (infinite ones) go element by element
+
+struct PolyBlock {
+  float X, Y;    // the block's middle
+  float sx, sy;  // scales (powers of two)
+  float fx, fy;  // max |xi|, max |eta|
+  int ex, ey;    // log2 of the scales
+};
+
+__device__ inline float row16_max(float v) {  // over each row of 16 lanes, in every lane
+  v = fmaxf(v, dpp_f32<0xb1>(v));
+  v = fmaxf(v, dpp_f32<0x4e>(v));
+  v = fmaxf(v, dpp_f32<0x141>(v));
+  return fmaxf(v, dpp_f32<0x140>(v));
+}
+
+__device__ inline PolyBlock poly_block(const Problem& p, const float* __restrict__ row_coords,
+                                       const float* __restrict__ col_coords, int32_t r0, int32_t c0) {
+  const int l16 = threadIdx.x & 15;
+  PolyBlock k;
+  k.X = row_coords[min(r0 + 8, p.M - 1)];
+  k.Y = col_coords[min(c0 + 8, p.N - 1)];
+  const float xd = row_coords[min(r0 + l16, p.M - 1)] - k.X, yd = col_coords[min(c0 + l16, p.N - 1)] - k.Y;
+  const float hx = readlane_f(row16_max(fabsf(xd)), 0), hy = readlane_f(row16_max(fabsf(yd)), 0);  // uniform
+  const int ex = __builtin_amdgcn_frexp_expf(hx), ey = __builtin_amdgcn_frexp_expf(hy);
+  k.sx = ldexpf(1.0f, ex);
+  k.sy = ldexpf(1.0f, ey);
+  k.fx = ldexpf(hx, -ex);
+  k.fy = ldexpf(hy, -ey);
+  k.ex = ex;
+  k.ey = ey;
+  return k;
+}
+
+// A Gaussian's exponent about a block, and whether the polynomial stands for it there.
+struct PolyGauss {
+  float L1, L2, Q11x2, Q12, Q22x2, e0;
+  bool wide;
+};
+__device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
+#pragma clang fp contract(off)
+  constexpr float ln2 = 0.69314718055994530942f;
+  PolyGauss o;
+  const float dx = k.X - u.mu0, dy = k.Y - u.mu1;
+  const float a0 = u.wa * dx, z0 = __builtin_fmaf(u.wc, dy, u.wb * dx);
+  const float al = u.wa * k.sx, be = u.wb * k.sx, ga = u.wc * k.sy;
+  const float la = a0 * al, lb = z0 * be, lc = z0 * ga;
+  const float lin = (2.0f * ln2) * ((fabsf(la) + fabsf(lb)) * k.fx + fabsf(lc) * k.fy);
+  const float h = fabsf(be) * k.fx + fabsf(ga) * k.fy, v = al * k.fx;
+  // (comparisons that a NaN fails)
+  const float reach = lin + (8.0f * ln2) * (v * v + h * h);
+  const float q = __builtin_fmaf(z0, z0, a0 * a0);
+  o.wide = u.gen == 0.0f && reach <= kPolyReach * __builtin_amdgcn_exp2f(q * (1.0f / (kPolyDeg + 1))) &&
+           q <= kPolyMaxQ && fabsf(u.w) <= kPolyMaxAmp;
+  o.L1 = (2.0f * ln2) * (la + lb);
+  o.L2 = (2.0f * ln2) * lc;
+  o.Q11x2 = (2.0f * ln2) * (al * al + be * be);
+  o.Q12 = (2.0f * ln2) * (be * ga);
+  o.Q22x2 = (2.0f * ln2) * (ga * ga);
+  o.e0 = __builtin_amdgcn_exp2f(-q);
+  return o;
+}
+
+// The coefficients c_ab of c00 * e / e0, a-major, b ascending: emit(a, b, c_ab) for a + b <= D.
+template <int D, typename Emit>
+__device__ __forceinline__ void poly_coefs(const PolyGauss& o, float c00, Emit&& emit) {
+  float prev[D + 1], prev2[D + 1];
+#pragma unroll
+  for (int a = 0; a <= D; ++a) {
+    float cur[D + 1];
+    if (a == 0) {
+      cur[0] = c00;
+#pragma unroll
+      for (int b = 0; b < D; ++b) {
+        float v = (o.L2 * (-1.0f / (b + 1))) * cur[b];
+        if (b > 0) v = fmaf(o.Q22x2 * (-1.0f / (b + 1)), cur[b - 1], v);
+        cur[b + 1] = v;
+      }
+    } else {
+      const float n1 = o.L1 * (-1.0f / a), n2 = o.Q11x2 * (-1.0f / a), n3 = o.Q12 * (-1.0f / a);
+#pragma unroll
+      for (int b = 0; b <= D - a; ++b) {
+        float v = n1 * prev[b];
+        if (a > 1) v = fmaf(n2, prev2[b], v);
+        if (b > 0) v = fmaf(n3, prev[b - 1], v);
+        cur[b] = v;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b <= D - a; ++b) emit(a, b, cur[b]);
+#pragma unroll
+    for (int b = 0; b <= D - a; ++b) {
+      prev2[b] = a > 0 ? prev[b] : 0.0f;
+      prev[b] = cur[b];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // a row at a time: the rows ahead would hold registers
+  }
+}
+
+constexpr int kPolyCoefs = (kPolyDeg + 1) * (kPolyDeg + 2) / 2;  // 45
+constexpr int kPolyRegs = 6;
+static_assert(kPolyDeg == 8, "the places below are those of 45 coefficients in 6 registers");
+
+// The block's sums of the coefficients over the wave's lanes, as they come: register q holds coefficients
+// 8 q + {0, 2, 1, 3} in lanes 0..7 of lane rows 0..3 (of 16 lanes) and 8 q + 4 + {0, 2, 1, 3} in lanes 8..15,
+// each still spread over its eight lanes.
+struct PolySum {
+  float r[kPolyRegs];
+};
+
+__device__ __forceinline__ void poly_sum_add(PolySum& ps, const PolyGauss& o, float c00) {
+  float q[4], lo = 0.0f;
+  poly_coefs<kPolyDeg>(o, c00, [&](int a, int b, float c) {
+    const int i = a * (kPolyDeg + 1) - a * (a - 1) / 2 + b;  // the coefficient's place in the order
+    q[i & 3] = c;
+    const bool last = i == kPolyCoefs - 1;  // place 44, the first of its four
+    if ((i & 3) != 3 && !last) return;
+    const float v = swap16_add(swap32_add(q[0], last ? 0.0f : q[1]), last ? 0.0f : swap32_add(q[2], q[3]));
+    if ((i & 4) == 0) {
+      lo = dpp_f32<0x140>(v) + v;
+      if (last) ps.r[i >> 3] += lo;  // (not reached: place 44 is in the upper four)
+    } else {
+      ps.r[i >> 3] += row_mirror_sum_upper(lo, v);
+    }
+  });
+}
+
+// The polynomial of the sums at the lane's elements: row lane / 4, columns 4 (lane % 4) .. + 3, whose offsets
+// xi (row) and eta (columns) are given.  lds: 128 floats of the wave's.
+__device__ __forceinline__ void poly_eval(const PolySum& ps, float xi, const float (&eta)[4], float* lds, float (&out)[4]) {
+  const int lane = threadIdx.x & 63;
+  const bool hb0 = (lane & 1) != 0, hb1 = (lane & 2) != 0;
+  // each register over its rows' lanes by recursive halving (as the backward's moments): lane bits
+  // 3, 2, 1 pick registers (in units of four places) 4 b1 + 2 b2 + b3 in even lanes, 8 + 2 b2 + b3 in odd ones
+  float q[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    q[i] = row_half_mirror_sum_odd_banks(dpp_f32<0x141>(ps.r[2 * i]) + ps.r[2 * i], ps.r[2 * i + 1]);
+  const float m0 = (hb1 ? q[1] : q[0]) + dpp_f32<0x4e>(hb1 ? q[0] : q[1]);
+  const float m1 = q[2] + dpp_f32<0x4e>(q[2]);
+  const float own = (hb0 ? m1 : m0) + dpp_f32<0xb1>(hb0 ? m0 : m1);
+  const int reg = ((lane >> 3) & 1) + ((lane >> 1) & 2) + (hb0 ? 8 : (hb1 ? 4 : 0));
+  const int grp = lane >> 4;
+  const int idx = 4 * reg + ((grp >> 1) | ((grp & 1) << 1));
+  int a = 0, first = 0;  // the a of the c_ab at place idx
+#pragma unroll
+  for (int i = 1; i <= kPolyDeg; ++i) {
+    const int st = i * (kPolyDeg + 1) - i * (i - 1) / 2;
+    a = idx >= st ? i : a;
+    first = idx >= st ? st : first;
+  }
+  if (idx < kPolyCoefs) lds[12 * (idx - first) + a] = own;  // [b][a], rows of 12
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) out[i] = 0.0f;
+#pragma unroll
+  for (int b = kPolyDeg; b >= 0; --b) {
+    float t = 0.0f;
+#pragma unroll
+    for (int a4 = (kPolyDeg - b) / 4; a4 >= 0; --a4) {
+      const f32x4_t c = *reinterpret_cast<const f32x4_t*>(lds + 12 * b + 4 * a4);
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        const int aa = 4 * a4 + j;
+        if (aa <= kPolyDeg - b) t = aa == kPolyDeg - b ? c[j] : fmaf(t, xi, c[j]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = b == kPolyDeg ? t : fmaf(out[i], eta[i], t);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  wave_sync();
+}
+
 // ------------------------------------------------------------------------------------------
 // Forward render.
 
@@ -1697,6 +1910,8 @@ __shared__ float4 r16_wevals[kTileThreads / 64][128];
 constexpr int kRowsThreads = 512;
 __shared__ float4 r16_rows_wevals[kRowsThreads / 64][128];
 
+constexpr int32_t kWideKey = 1 << 30;  // a key whose Gaussian the block's polynomial holds
+
 __device__ __forceinline__ void render16_body(
     const Problem& p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr, int64_t* ids,
@@ -1783,10 +1998,13 @@ __device__ __forceinline__ void render16_body(
   // Gaussians.
   auto& wevals = r16_wevals;
   float4* ew = wevals[wid];
-  auto run_chunk = [&](const GaussEval& my, int nj) {
+  // (si: the lane's place among the chunk's Gaussians, negative for none)
+  auto run_chunk = [&](const GaussEval& my, int nj, int si) {
     // two arrays of 64 float4 (conflict-free writes, broadcast reads)
-    ew[lane] = make_float4(my.mu0, my.mu1, my.wa, my.wb);
-    ew[64 + lane] = make_float4(my.wc, my.w, __int_as_float(my.gid), my.gen);
+    if (si >= 0) {
+      ew[si] = make_float4(my.mu0, my.mu1, my.wa, my.wb);
+      ew[64 + si] = make_float4(my.wc, my.w, __int_as_float(my.gid), my.gen);
+    }
     wave_sync();
     auto at = [&](int j) {
       const float4 a = ew[j], b = ew[64 + j];
@@ -1801,7 +2019,7 @@ __device__ __forceinline__ void render16_body(
       u.gen = b.w;
       return u;
     };
-    if (__builtin_amdgcn_ballot_w64(lane < nj && my.gen != 0.0f) == 0) {
+    if (__builtin_amdgcn_ballot_w64(si >= 0 && my.gen != 0.0f) == 0) {
       if (floor_free)
         for (int j = 0; j < nj; ++j) accumulate_free(at(j));
       else
@@ -1911,11 +2129,53 @@ __device__ __forceinline__ void render16_body(
             if (slot < room) ids[s + slot] = keys[j];
           }
         }
+        // The window's wide Gaussians as one polynomial, 64 at a time where enough of them are; they are
+        // marked in their keys and left out below.
+        bool marked = false;
+        if (F == 1 && floor_free && nwin >= kPolyMin) {
+          const PolyBlock pb = poly_block(p, row_coords, col_coords, st.r0, st.c0);
+          PolySum ps;
+          for (int32_t j0 = 0; j0 < nwin; j0 += 64) {
+            const bool mine = lane < min(64, nwin - j0);
+            const int32_t key = mine ? keys[j0 + lane] : 0;
+            GaussEval my = zero_eval();
+            if (mine) my = load_eval(ev, key);
+            const PolyGauss g = poly_gauss(pb, my);
+            const bool wide = mine && g.wide;
+            const int nw = __popcll(__builtin_amdgcn_ballot_w64(wide));
+            if (nw < (marked ? kPolyMore : kPolyMin)) continue;  // wave-uniform
+            if (!marked) {
+#pragma unroll
+              for (int i = 0; i < kPolyRegs; ++i) ps.r[i] = 0.0f;
+              marked = true;
+            }
+            poly_sum_add(ps, g, wide ? my.w * g.e0 : 0.0f);
+            if (wide) keys[j0 + lane] = key | kWideKey;
+          }
+          if (marked) {
+            float eta[4], v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) eta[i] = ldexpf(col_coords[min(pc + i, p.N - 1)] - pb.Y, -pb.ey);
+            poly_eval(ps, ldexpf(x - pb.X, -pb.ex), eta, reinterpret_cast<float*>(ew), v);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] += v[i];
+          }
+        }
         for (int32_t j0 = q * cs; j0 < nwin; j0 += F * cs) {
           const int nj = min(cs, nwin - j0);
           GaussEval my = zero_eval();
-          if (lane < nj) my = load_eval(ev, keys[j0 + lane]);
-          run_chunk(my, nj);
+          const int32_t key = lane < nj ? keys[j0 + lane] : kWideKey;
+          if (marked) {
+            const bool mine = (key & kWideKey) == 0;
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(mine);
+            if (bal == 0ull) continue;  // wave-uniform
+            if (mine) my = load_eval(ev, key);
+            run_chunk(my, __popcll(bal), mine ? (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u)) : -1);
+          } else {
+            if (lane < nj) my = load_eval(ev, key);
+            run_chunk(my, nj, lane < nj ? lane : -1);
+          }
         }
         done += nwin;
         wave_sync();
@@ -1954,7 +2214,7 @@ __device__ __forceinline__ void render16_body(
       if (srt.gid < 0 || srt.gid >= p.K) set_status(&hdr->status, GF_STATUS_COUNT_MISMATCH);
       if (srt.gid != key) ids[s + lane] = srt.gid;  // lanes whose id moved
     }
-    run_chunk(srt, (int)n);
+    run_chunk(srt, (int)n, lane < n ? lane : -1);
   } else if (n > 64) {
     int64_t* seg = ids + s;
     int32_t* keys = wkeys[wid];
@@ -1970,7 +2230,7 @@ __device__ __forceinline__ void render16_body(
           set_status(&hdr->status, GF_STATUS_COUNT_MISMATCH);  // internal mismatch only
         }
       }
-      run_chunk(my, nj);
+      run_chunk(my, nj, lane < nj ? lane : -1);
     }
   }
   if (F > 1) {
@@ -2472,7 +2732,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
 }
 
 template <bool kHeavy>
-__global__ __launch_bounds__(kTileThreads) void k_render16(
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_render16(
     Problem p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr, int64_t* ids,
     int64_t capacity, float* __restrict__ delta, uint8_t* ws, const uint32_t* __restrict__ rowmask,
@@ -3047,19 +3307,6 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
 // delta-W therefore sums each pixel's Gaussians in a different order than the render (four
 // interleaved partial sums): within fp32 rounding of it, not bit-equal.
 constexpr int kFusedKeys = 128;  // ids expanded per window (a tile of more takes several windows)
-
-// Lanes 0..31 of the result: a + (a of lane + 32); lanes 32..63: (b of lane - 32) + b
-// (v_permlane32_swap exchanges lanes 32..63 of its first operand with lanes 0..31 of its second).
-__device__ inline float swap32_add(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-// Rows of 16 lanes: row 2i + 0 of the result: a + (a of lane + 16); row 2i + 1: (b of lane - 16) + b
-// (v_permlane16_swap exchanges the odd rows of its first operand with the even rows of its second).
-__device__ inline float swap16_add(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 // kRows (rows_in_render fields): a workgroup of kRowsThreads takes eight tiles of one tile row
 // (ceil(C / 8) workgroups a row), bins that row first (bin_tile_row: no k_bin_tiles launch,
@@ -3902,7 +4149,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_batch(const uint8_t* __re
 
 // Layers rendered tile by tile (BatchLayer::pair_render == 0: 32x32 tiles, or 16x16 tiles whose
 // capacity reaches the emission path), over the tile map; the other layers' blocks return.
-__global__ __launch_bounds__(kTileThreads) void k_render16_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_render16_batch(const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   const uint32_t blk = blockIdx.x;

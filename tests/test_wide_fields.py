@@ -61,3 +61,60 @@ def test_striped_reduction_of_few_gaussians(M, Nf, K, tile, device):
                                           forward_workspace=fws)
         for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), got, r[3:]):
             grad_close(a, b, name)
+
+
+def _mixed(M: int, Nf: int, K: int, seed: int) -> wl.FieldProblem:
+    """init_problem with every fifth Gaussian a few elements wide, listed between the others."""
+    p = init_problem(M, Nf, K, seed)
+    sub = p.chol_raw[::5]
+    p.chol_raw[::5] = torch.stack((torch.full_like(sub[:, 0], math.log(math.expm1(8.0 / M))), torch.zeros_like(sub[:, 1]),
+                                   torch.full_like(sub[:, 2], math.log(math.expm1(8.0 / Nf)))), dim=-1)
+    return p
+
+
+# Blocks cut by the matrix's edges, one row and one column of blocks, lists of 24 (the fewest taken), 64, 65 and
+# several times 64, narrow Gaussians between the wide ones, normalised ones, and a clamp that keeps them all
+# element by element.
+WIDE_CASES = {
+    "ragged": (250, 333, 200, 32, {}),
+    "one_row": (9, 700, 60, 16, {}),
+    "n24": (64, 64, 24, 16, {}),
+    "n64": (64, 80, 64, 32, {}),
+    "n65": (80, 64, 65, 32, {}),
+    "mixed": (330, 200, 150, 32, {}),
+    "normalize": (128, 200, 90, 16, {"normalize": True}),
+    "clamp24": (128, 200, 90, 32, {"clamp": 24.0}),
+    "noclamp": (200, 128, 256, 16, {"clamp": None}),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", list(WIDE_CASES))
+def test_wide_gaussians_render(case, device):
+    """Blocks of wide Gaussians as polynomials against the oracle's exponentials, at the parity bar."""
+    from guass_amd.cuda_field import ext
+    from oracle import field_oracle as fo
+
+    M, Nf, K, tile, kw = WIDE_CASES[case]
+    p = (_mixed if case == "mixed" else init_problem)(M, Nf, K, 7, **({} if case == "mixed" else {"sigma": max(3.0 / math.sqrt(K), 0.7)}))
+    norm, clamp = kw.get("normalize", False), kw.get("clamp", 80.0)
+    r = fo.gaussian_field_fwd_bwd_batched(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, tile, tile,
+                                          3.0, norm, clamp)
+    q = p.to(device)
+    delta, tp, ids = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tile, tile, 3.0,
+                                                norm, clamp)
+    binning_equal(tp, ids, r[1], r[2])
+    field_close(delta, r[0])
+
+
+@pytest.mark.gpu
+def test_wide_gaussians_infinite_amplitude(device):
+    """An infinite amplitude among wide Gaussians stays out of the block's polynomial: every element it
+    reaches is infinite, not NaN."""
+    from guass_amd.cuda_field import ext
+
+    p = init_problem(64, 64, 64, 3, sigma=1.5)
+    p.amp[10] = float("inf")
+    q = p.to(device)
+    delta, _, _ = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, 32, 32, 3.0, False, 80.0)
+    assert torch.isposinf(delta).all()
