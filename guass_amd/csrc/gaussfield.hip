@@ -163,7 +163,8 @@ struct __align__(16) GaussEval {
 
 struct WsHeader {
   uint32_t status;
-  uint32_t heavy;      // forward, heavy-tile mode: tiles in the heavy-tile list
+  uint32_t heavy;      // forward, heavy-tile mode: tiles in the heavy-tile list; backward: k_bwd_wide left
+                       // Gaussians to k_bwd_rest
   int64_t* num_pairs;  // forward, tiles binned in the render: where the render stores P
   int64_t pairs;       // forward: P as the binning computed it, beside the status word, so that
                        // one 32-byte copy reads both back (gf_forward_bin's num_pairs_host)
@@ -1609,6 +1610,13 @@ __device__ inline float swap16_add(float a, float b) {
 }
 
 
+// The lane, opaque: what a loop over blocks derives from it is computed anew, not held in registers across it.
+__device__ inline int opaque_lane() {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 // ------------------------------------------------------------------------------------------
 // Wide Gaussians: one whose exponent changes little over a 16x16 block is a short polynomial there.
 // About the block's middle (X, Y), with xi = (x - X) / sx and eta = (y - Y) / sy (sx, sy powers of
@@ -1629,6 +1637,9 @@ __device__ inline float swap16_add(float a, float b) {
 // 64 lanes' terms add in a tree, and one exponential's argument is rounded instead of 256.
 constexpr int kPolyDeg = 8;
 constexpr float kPolyReach = 0.85f;
+// Where it holds for every Gaussian of the 64, degree 6 does (28 coefficients): 1.5e-6 along l + 8 k = 0.5.
+constexpr int kPolyShort = 6;
+constexpr float kPolyShortReach = 0.5f;
 // Fewer wide Gaussians than this in 64 do not repay the reduction and the evaluation (about 450
 // instructions a block against 24-34 a Gaussian).
 constexpr int kPolyMin = 24;
@@ -1652,7 +1663,7 @@ __device__ inline float row16_max(float v) {  // over each row of 16 lanes, in e
 
 __device__ inline PolyBlock poly_block(const Problem& p, const float* __restrict__ row_coords,
                                        const float* __restrict__ col_coords, int32_t r0, int32_t c0) {
-  const int l16 = threadIdx.x & 15;
+  const int l16 = opaque_lane() & 15;
   PolyBlock k;
   k.X = row_coords[min(r0 + 8, p.M - 1)];
   k.Y = col_coords[min(c0 + 8, p.N - 1)];
@@ -1671,7 +1682,8 @@ __device__ inline PolyBlock poly_block(const Problem& p, const float* __restrict
 // A Gaussian's exponent about a block, and whether the polynomial stands for it there.
 struct PolyGauss {
   float L1, L2, Q11x2, Q12, Q22x2, e0;
-  bool wide;
+  bool wide;   // degree kPolyDeg stands for it
+  bool short_; // so does degree kPolyShort
 };
 __device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
 #pragma clang fp contract(off)
@@ -1688,6 +1700,7 @@ __device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
   const float q = __builtin_fmaf(z0, z0, a0 * a0);
   o.wide = u.gen == 0.0f && reach <= kPolyReach * __builtin_amdgcn_exp2f(q * (1.0f / (kPolyDeg + 1))) &&
            q <= kPolyMaxQ && fabsf(u.w) <= kPolyMaxAmp;
+  o.short_ = o.wide && reach <= kPolyShortReach * __builtin_amdgcn_exp2f(q * (1.0f / (kPolyShort + 1)));
   o.L1 = (2.0f * ln2) * (la + lb);
   o.L2 = (2.0f * ln2) * lc;
   o.Q11x2 = (2.0f * ln2) * (al * al + be * be);
@@ -1697,36 +1710,36 @@ __device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
   return o;
 }
 
-// The coefficients c_ab of c00 * e / e0, a-major, b ascending: emit(a, b, c_ab) for a + b <= D.
+// The coefficients c_ab of c00 * e / e0, a + b <= D, a-major: emit(a, b, c_a, c_{a-1}, c_{a-2}), rows indexed by b,
+// is called as c_ab is computed (c_a so far; the rows before are zero past the degree and before the first).
 template <int D, typename Emit>
 __device__ __forceinline__ void poly_coefs(const PolyGauss& o, float c00, Emit&& emit) {
   float prev[D + 1], prev2[D + 1];
 #pragma unroll
+  for (int b = 0; b <= D; ++b) prev[b] = prev2[b] = 0.0f;
+#pragma unroll
   for (int a = 0; a <= D; ++a) {
     float cur[D + 1];
-    if (a == 0) {
-      cur[0] = c00;
-#pragma unroll
-      for (int b = 0; b < D; ++b) {
-        float v = (o.L2 * (-1.0f / (b + 1))) * cur[b];
-        if (b > 0) v = fmaf(o.Q22x2 * (-1.0f / (b + 1)), cur[b - 1], v);
-        cur[b + 1] = v;
-      }
-    } else {
-      const float n1 = o.L1 * (-1.0f / a), n2 = o.Q11x2 * (-1.0f / a), n3 = o.Q12 * (-1.0f / a);
-#pragma unroll
-      for (int b = 0; b <= D - a; ++b) {
-        float v = n1 * prev[b];
-        if (a > 1) v = fmaf(n2, prev2[b], v);
-        if (b > 0) v = fmaf(n3, prev[b - 1], v);
-        cur[b] = v;
-      }
-    }
-#pragma unroll
-    for (int b = 0; b <= D - a; ++b) emit(a, b, cur[b]);
+    const float n1 = a > 0 ? o.L1 * (-1.0f / (a > 0 ? a : 1)) : 0.0f, n2 = a > 1 ? o.Q11x2 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
+    const float n3 = a > 0 ? o.Q12 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
 #pragma unroll
     for (int b = 0; b <= D - a; ++b) {
-      prev2[b] = a > 0 ? prev[b] : 0.0f;
+      float v;
+      if (a == 0) {
+        v = c00;
+        if (b > 0) v = (o.L2 * (-1.0f / (b > 0 ? b : 1))) * cur[b - 1];
+        if (b > 1) v = fmaf(o.Q22x2 * (-1.0f / (b > 0 ? b : 1)), cur[b - 2], v);
+      } else {
+        v = n1 * prev[b];
+        if (a > 1) v = fmaf(n2, prev2[b], v);
+        if (b > 0) v = fmaf(n3, prev[b - 1], v);
+      }
+      cur[b] = v;
+      emit(a, b, cur, prev, prev2);
+    }
+#pragma unroll
+    for (int b = 0; b <= D - a; ++b) {
+      prev2[b] = prev[b];
       prev[b] = cur[b];
     }
     __builtin_amdgcn_sched_barrier(0);  // a row at a time: the rows ahead would hold registers
@@ -1746,18 +1759,16 @@ struct PolySum {
 
 __device__ __forceinline__ void poly_sum_add(PolySum& ps, const PolyGauss& o, float c00) {
   float q[4], lo = 0.0f;
-  poly_coefs<kPolyDeg>(o, c00, [&](int a, int b, float c) {
+  poly_coefs<kPolyDeg>(o, c00, [&](int a, int b, const float* cur, const float*, const float*) {
     const int i = a * (kPolyDeg + 1) - a * (a - 1) / 2 + b;  // the coefficient's place in the order
-    q[i & 3] = c;
-    const bool last = i == kPolyCoefs - 1;  // place 44, the first of its four
+    q[i & 3] = cur[b];
+    const bool last = i == kPolyCoefs - 1;  // place 44, the first of its four, in the upper half of a register
     if ((i & 3) != 3 && !last) return;
     const float v = swap16_add(swap32_add(q[0], last ? 0.0f : q[1]), last ? 0.0f : swap32_add(q[2], q[3]));
-    if ((i & 4) == 0) {
+    if ((i & 4) == 0)
       lo = dpp_f32<0x140>(v) + v;
-      if (last) ps.r[i >> 3] += lo;  // (not reached: place 44 is in the upper four)
-    } else {
+    else
       ps.r[i >> 3] += row_mirror_sum_upper(lo, v);
-    }
   });
 }
 
@@ -2846,6 +2857,80 @@ __device__ inline void stage_gaussians(const Problem& p, const GIdx* __restrict_
   }
 }
 
+// The backward's side of the polynomial form (poly_coefs).
+//
+// M[a][b] = sum over a block of dL/d(delta-W) xi^a eta^b, a + b <= kPolyDeg, as two products of 16x16 matrices on
+// the matrix cores (fp32): R = G Vy, then M = Vx^T R.  gt: the block's dL/d(delta-W), rows of kWideRow floats; pw:
+// 288 floats for the powers; M: rows of 12.
+constexpr int kWideRow = 20;
+constexpr int kPolyM = 12 * (kPolyDeg + 1);
+__device__ __forceinline__ void poly_moments(const Problem& p, const PolyBlock& k, const float* __restrict__ row_coords,
+                                             const float* __restrict__ col_coords, int32_t r0, int32_t c0,
+                                             const float* gt, float* pw, float* M) {
+  const int lane = opaque_lane(), l16 = lane & 15, grp = lane >> 4;
+  if (lane < 32) {  // xi_i^e at [e][i], eta_i^e at [e][16 + i]
+    const float v = grp == 0 ? ldexpf(row_coords[min(r0 + l16, p.M - 1)] - k.X, -k.ex)
+                             : ldexpf(col_coords[min(c0 + l16, p.N - 1)] - k.Y, -k.ey);
+    float e = 1.0f;
+#pragma unroll
+    for (int i = 0; i <= kPolyDeg; ++i) {
+      pw[32 * i + lane] = e;
+      e *= v;
+    }
+  }
+  wave_sync();
+  const int e = min(l16, kPolyDeg);  // (lanes past the degree repeat it, and are not stored)
+  const float* px = pw + 32 * e;
+  const float* py = px + 16;
+  f32x4_t r = {0.f, 0.f, 0.f, 0.f}, m = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+    r = __builtin_amdgcn_mfma_f32_16x16x4f32(gt[kWideRow * l16 + 4 * s + grp], py[4 * s + grp], r, 0, 0, 0);
+  // r[i]: row 4 grp + i, b = l16; the second product contracts the rows in that order
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = __builtin_amdgcn_mfma_f32_16x16x4f32(px[4 * grp + i], r[i], m, 0, 0, 0);
+  // m[i]: a = 4 grp + i, b = l16
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int a = 4 * grp + i;
+    if (a + l16 <= kPolyDeg) M[12 * a + l16] = m[i];
+  }
+  wave_sync();
+}
+
+// Whether a block's dL/d(delta-W) (a float4 a lane) allows the polynomial form: not with an infinity, a NaN or
+// values near the overflow, which go element by element.
+__device__ inline bool poly_grad_fits(const float4& g) {
+  return __builtin_amdgcn_ballot_w64(!(fabsf(g.x) <= kPolyMaxAmp && fabsf(g.y) <= kPolyMaxAmp &&
+                                       fabsf(g.z) <= kPolyMaxAmp && fabsf(g.w) <= kPolyMaxAmp)) == 0ull;
+}
+// The six moments of the lane's Gaussian (about its mean) from the block's: sums of c_ab M[a + i][b + j] for
+// i + j <= 2 within the degree (each M read once, beside the rows it meets), shifted from the block's middle.
+template <int D>
+__device__ __forceinline__ void poly_six(const PolyBlock& k, const PolyGauss& o, const GaussEval& u, const float* M,
+                                         float (&m)[6]) {
+  float s00 = 0.f, s10 = 0.f, s01 = 0.f, s20 = 0.f, s11 = 0.f, s02 = 0.f;
+  f32x4_t v;
+  poly_coefs<D>(o, o.e0, [&](int a, int b, const float* cur, const float* prev, const float* prev2) {
+    if ((b & 3) == 0) v = *reinterpret_cast<const f32x4_t*>(M + 12 * a + b);
+    const float m_ab = v[b & 3];
+    s00 = fmaf(cur[b], m_ab, s00);
+    if (b > 0) s01 = fmaf(cur[b - 1], m_ab, s01);
+    if (b > 1) s02 = fmaf(cur[b - 2], m_ab, s02);
+    if (a > 0) s10 = fmaf(prev[b], m_ab, s10);
+    if (a > 0 && b > 0) s11 = fmaf(prev[b - 1], m_ab, s11);
+    if (a > 1) s20 = fmaf(prev2[b], m_ab, s20);
+  });
+  const float dx = k.X - u.mu0, dy = k.Y - u.mu1;
+  const float t10 = k.sx * s10, t01 = k.sy * s01;
+  m[0] = s00;
+  m[1] = fmaf(dx, s00, t10);
+  m[2] = fmaf(dy, s00, t01);
+  m[3] = fmaf(dx, m[1] + t10, (k.sx * k.sx) * s20);
+  m[4] = fmaf(dx, m[2], fmaf(dy, t10, (k.sx * k.sy) * s11));
+  m[5] = fmaf(dy, m[2] + t01, (k.sy * k.sy) * s02);
+}
+
 // 16x16 tiles, one wave per tile (tile blockIdx.x * 4 + wave).  Lane l: slot = l/16, row =
 // l%16; per round the four slots take four Gaussians of the tile and each lane sums its row's
 // 16 pixels.  Gaussian constants are computed one per lane for up to 64 Gaussians at a time
@@ -2854,7 +2939,7 @@ __device__ inline void stage_gaussians(const Problem& p, const GIdx* __restrict_
 // kEvalGiven: ev is never null (batches), so the per-Gaussian recomputation from mu / chol_raw
 // (the exact softplus chain) is left out of the kernel, with its registers.
 template <typename TpIdx, typename GIdx, bool kTransposeSums, bool kMaskClamp, bool kManyRounds = kTransposeSums,
-          bool kEvalGiven = false, bool kDirect = false>
+          bool kEvalGiven = false, bool kDirect = false, bool kRest = false>
 __device__ __forceinline__ void bwd16_body(
     const Problem& p, const float* __restrict__ grad, const float* __restrict__ row_coords,
     const float* __restrict__ col_coords, const float* __restrict__ mu,
@@ -2862,10 +2947,12 @@ __device__ __forceinline__ void bwd16_body(
     const TpIdx* __restrict__ tile_ptr, const GIdx* __restrict__ gids, int64_t num_pairs,
     uint8_t* ws, const BwdLayout& L, const SubTile& st, int q = 0, int F = 1,
     const float4* __restrict__ dcoef = nullptr, float* __restrict__ dgrad = nullptr) {
+  // kRest: the Gaussians that k_bwd_wide took (poly_gauss: the same test) are left out.  F == 1 only.
   // kDirect (row sums only): each tile's moments go through the Gaussian's chain-rule map
   // (dcoef, store_dcoef) and the gradients are added straight into the Gaussian's slot of dgrad
   // (direct_slot), so that no finish pass follows.
   static_assert(!kDirect || !kTransposeSums, "direct gradients take the row-sum reduction");
+  static_assert(!kRest || (kManyRounds && !kMaskClamp && kEvalGiven && !kDirect), "kRest: the dense-tile form");
   // F > 1 (heavy tiles): the F = 4 waves of the workgroup share tile st, wave q taking chunks
   // q, q + F, ... of kHeavyChunk Gaussians (and their indefinite-form pass).
   const int cs = F > 1 ? kHeavyChunk : 64;
@@ -2880,6 +2967,9 @@ __device__ __forceinline__ void bwd16_body(
   float* const acc_s = acc + 8 * acc_slot(p, 0, stripe);  // Gaussian 0's slot in this tile's stripe
   const bool hb3 = (lane & 8) != 0, hb2 = (lane & 4) != 0, hb1 = (lane & 2) != 0;
   const bool atomic_lane = (lane & 1) == 0 && (lane & 15) < 12;
+  auto add_moment = [&](int32_t g, int k, float v) {
+    unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)g + (uint32_t)k), v);
+  };
   const int slot = lane >> 4, row = lane & 15;
   const int32_t pr = r0 + row;
   // This lane's row of dL/d(delta) (0 outside the matrix) and the tile's coordinates are
@@ -2899,7 +2989,23 @@ __device__ __forceinline__ void bwd16_body(
   __shared__ float gtile[kTileThreads / 64][16 * 52];
   float* gt = gtile[__builtin_amdgcn_readfirstlane((int32_t)(threadIdx.x >> 6))];
   float gv[16], yv[16];
+  bool grad_fits = false;
   float ydl[4] = {0.f, 0.f, 0.f, 0.f};  // kShifted: the lane's four column offsets from column 8
+  // kShifted: the lane's share of the stage's other columns (and its four column offsets: lanes 0..3 hold the
+  // tile's 16, the scalar yd[] below).
+  auto stage_shifted = [&](const float4& g4) {
+    const int32_t lc = c0 + ((lane & 3) << 2);
+    float* gw = gt + (lane >> 2) * kGs + ((lane & 3) << 2);
+    const float yf = col_coords[min(c0 + 8, p.N - 1)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ydl[i] = col_coords[min(lc + i, p.N - 1)] - yf;
+    const float4 gy = make_float4(g4.x * ydl[0], g4.y * ydl[1], g4.z * ydl[2], g4.w * ydl[3]);
+    *reinterpret_cast<float4*>(gw + 16) = gy;
+    *reinterpret_cast<float4*>(gw + 32) = make_float4(gy.x * ydl[0], gy.y * ydl[1], gy.z * ydl[2], gy.w * ydl[3]);
+    // the 16 column offsets, a float4 per column group in the pad of rows 0..3, for the split
+    // rounds below (whose lanes take different columns)
+    if (lane < 4) *reinterpret_cast<float4*>(gt + lane * kGs + 48) = make_float4(ydl[0], ydl[1], ydl[2], ydl[3]);
+  };
   {
     const int32_t lr = r0 + (lane >> 2), lc = c0 + ((lane & 3) << 2);
     const float* gp = grad + (int64_t)min(lr, p.M - 1) * p.N + lc;
@@ -2921,20 +3027,9 @@ __device__ __forceinline__ void bwd16_body(
         g4.w = lc + 3 < p.N ? load_stream(gp + 3) : 0.f;
       }
     }
-    float* gw = gt + (lane >> 2) * kGs + ((lane & 3) << 2);
-    *reinterpret_cast<float4*>(gw) = g4;
-    if (kShifted) {
-      // the lane's four column offsets (lanes 0..3 hold the tile's 16, the scalar yd[] below)
-      const float yf = col_coords[min(c0 + 8, p.N - 1)];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ydl[i] = col_coords[min(lc + i, p.N - 1)] - yf;
-      const float4 gy = make_float4(g4.x * ydl[0], g4.y * ydl[1], g4.z * ydl[2], g4.w * ydl[3]);
-      *reinterpret_cast<float4*>(gw + 16) = gy;
-      *reinterpret_cast<float4*>(gw + 32) = make_float4(gy.x * ydl[0], gy.y * ydl[1], gy.z * ydl[2], gy.w * ydl[3]);
-      // the 16 column offsets, a float4 per column group in the pad of rows 0..3, for the split
-      // rounds below (whose lanes take different columns)
-      if (lane < 4) *reinterpret_cast<float4*>(gt + lane * kGs + 48) = make_float4(ydl[0], ydl[1], ydl[2], ydl[3]);
-    }
+    *reinterpret_cast<float4*>(gt + (lane >> 2) * kGs + ((lane & 3) << 2)) = g4;
+    if (kRest) grad_fits = poly_grad_fits(g4);
+    if (kShifted) stage_shifted(g4);
     wave_sync();
     if (!kShifted) {
 #pragma unroll
@@ -2962,13 +3057,6 @@ __device__ __forceinline__ void bwd16_body(
 #pragma unroll
     for (int c = 0; c < 16; ++c) yv[c] = col_coords[min(c0 + c, p.N - 1)];
   }
-  // kShifted: columns as offsets from the tile's middle one, column 8 (uniform: scalar
-  // registers), for the moments about that column below: column c's is lane c / 4's ydl[c % 4].
-  float yd[16];
-#pragma unroll
-  for (int c = 0; c < 16; ++c)
-    yd[c] = kShifted ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ydl[c & 3]), c >> 2)) : 0.0f;
-  const float x = row_coords[min(pr, p.M - 1)];
   int64_t s = (int64_t)tile_ptr[t], e = (int64_t)tile_ptr[t + 1];
   num_pairs = live_pairs(p, num_pairs);
   const int64_t Kl = live_k(p);
@@ -2982,9 +3070,16 @@ __device__ __forceinline__ void bwd16_body(
   if (n == 0) return;
   if (F == 1 && p.heavy > 0 && n > p.heavy) return;  // a heavy-tile workgroup's
 
+  PolyBlock pb;
+  if constexpr (kRest) pb = poly_block(p, row_coords, col_coords, r0, c0);
+  const float x = row_coords[min(pr, p.M - 1)];
+  float yd[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c)
+    yd[c] = kShifted ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ydl[c & 3]), c >> 2)) : 0.0f;
   bool tile_general = false;
   for (int64_t j0 = q * cs; j0 < n; j0 += F * cs) {
-    const int nj = (int)((n - j0) < cs ? (n - j0) : cs);
+    int nj = (int)((n - j0) < cs ? (n - j0) : cs);
     GaussEval my = zero_eval();
     int32_t myg = -1;
     if (lane < nj) {
@@ -2995,6 +3090,23 @@ __device__ __forceinline__ void bwd16_body(
         my = (kEvalGiven || ev) ? load_eval(ev, g) : eval_geom(p, mu, chol_raw, nullptr, g);
         myg = (int32_t)g;
       }
+    }
+    const uint64_t skip = kRest && grad_fits ? __builtin_amdgcn_ballot_w64(myg >= 0 && poly_gauss(pb, my).wide) : 0ull;
+    if (kRest && skip != 0ull) {
+      // the others to the front, in order
+      const bool rest = ((skip >> lane) & 1ull) == 0 && lane < nj;
+      const uint64_t rbal = __builtin_amdgcn_ballot_w64(rest);
+      nj = __popcll(rbal);
+      const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(rbal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)rbal, 0u));
+      const int to = (rest ? below : nj + lane - below) << 2;
+      auto send = [&](float f) { return __int_as_float(__builtin_amdgcn_ds_permute(to, __float_as_int(f))); };
+      my.mu0 = send(my.mu0);
+      my.mu1 = send(my.mu1);
+      my.wa = send(my.wa);
+      my.wb = send(my.wb);
+      my.wc = send(my.wc);
+      my.gen = send(my.gen);
+      myg = __builtin_amdgcn_ds_permute(to, myg);
     }
     const bool chunk_general = __builtin_amdgcn_ballot_w64(lane < nj && my.gen != 0.0f) != 0;
     // kShifted: a last round of one or two Gaussians splits their columns over the four slots
@@ -3148,11 +3260,10 @@ __device__ __forceinline__ void bwd16_body(
           float val = k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : k == 3 ? v3 : k == 4 ? v4 : s5;
           val += __shfl_xor(val, 16, 64);
           if (rem == 1) val += __shfl_xor(val, 32, 64);
-          if (g >= 0 && row >= 10 && part == 0)
-            unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)g + (uint32_t)k), val);
+          if (g >= 0 && row >= 10 && part == 0) add_moment(g, k, val);
         } else if (g >= 0 && row >= 10) {
           const float val = k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : k == 3 ? v3 : k == 4 ? v4 : s5;
-          unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)g + (uint32_t)k), val);
+          add_moment(g, k, val);
         }
         continue;
       }
@@ -3183,8 +3294,7 @@ __device__ __forceinline__ void bwd16_body(
         d += __shfl_xor(d, 16, 64);
         if (rem == 1) d += __shfl_xor(d, 32, 64);
       }
-      if (g >= 0 && atomic_lane && part == 0)
-        unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)g + (uint32_t)(row >> 1)), d);
+      if (g >= 0 && atomic_lane && part == 0) add_moment(g, row >> 1, d);
     }
     }
     tile_general = tile_general || chunk_general;
@@ -3250,7 +3360,7 @@ __device__ __forceinline__ void bwd16_body(
           } else {
 #pragma unroll
             for (int k = 0; k < 6; ++k)
-              unsafeAtomicAdd(acc + 8 * acc_slot(p, gj, stripe) + k, mm[k]);
+              add_moment(gj, k, mm[k]);
           }
         }
       }
@@ -3283,6 +3393,257 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
   bwd16_body<TpIdx, GIdx, kTransposeSums, kMaskClamp, kTransposeSums || kHeavy, kEvalGiven, kDirect>(
       p, grad, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gids, num_pairs, ws, L, it.st, it.q, it.F,
       dcoef, dgrad);
+}
+
+// Fields of wide Gaussians (wide_field).  k_bwd_wide takes four blocks a wave -- a 32x32 tile's quadrants, or 2x2 tiles
+// of 16x16 -- with a listed Gaussian a lane: the four blocks' moments of dL/d(delta-W) first (poly_moments), then
+// 64 Gaussians of the blocks' lists at a time, each lane's six moments summed over the blocks where its Gaussian is
+// wide (poly_six) and added once.  What is not wide somewhere, k_bwd_rest takes block by block (it returns at once
+// where the workspace's flag says that nothing is left).
+//
+// Device-wide float atomics run at about 160 lanes' adds a nanosecond on the whole chip here: 11 million of
+// them (six a Gaussian and block) held a 1280x5120 field of 1024 wide Gaussians at 120 us in a form with a block a
+// wave, where the same kernel without its atomics took 50; four blocks' sums make a quarter of the adds.
+// Reductions, element by element -> this and the rest: that field 176 -> 56 us, 1280x1280 K = 256 on 32x32 tiles
+// 37 -> 22 us, 28 layers of K = 256 366 -> 105 us (all of it was 743 -> 267 us with the render's polynomials).
+constexpr int kWideKeys = 256;
+struct WideLds {            // a wave's
+  float gt[16 * kWideRow];  // a block's dL/d(delta-W); later the moments on their way out
+  float pw[32 * (kPolyDeg + 1)];
+  float M[4][kPolyM];
+  float block[4][8];  // PolyBlock's X, Y, sx, sy, fx, fy
+  int32_t keys[kWideKeys];
+};
+
+// Lists of kPolyMin Gaussians or more a tile on average, each over kWideBlocks blocks or more (a side of fourteen
+// blocks: a sigma of about 35 elements, poly_gauss's reach), on the masks' K.
+constexpr int64_t kWideBlocks = 192;
+// Single fields of fewer blocks leave most SIMDs without one of these longer waves: 320x320 (400 blocks), K = 32 took
+// 12.8 us against 8.5 for a block a wave.  In a batch the other layers fill them.
+constexpr int64_t kWideMinBlocks = 2048, kWideBatchMinBlocks = 256;
+__host__ __device__ inline bool wide_field(const Problem& p, int64_t pairs, int64_t min_blocks = kWideMinBlocks) {
+  const int64_t q = p.tile_out == 32 && p.tile_in == 32 ? 4 : 1;
+  return ((p.tile_out == 16 && p.tile_in == 16) || q == 4) && !p.mask_clamp && p.K >= 1 && p.K <= kMaskMaxK &&
+         q * p.R * p.C >= min_blocks && pairs >= kPolyMin * (int64_t)p.R * p.C && q * pairs >= kWideBlocks * p.K;
+}
+
+template <bool kQuad>
+__device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __restrict__ grad,
+                                              const float* __restrict__ row_coords,
+                                              const float* __restrict__ col_coords,
+                                              const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr,
+                                              const int64_t* __restrict__ gids, int64_t num_pairs, uint8_t* ws,
+                                              const BwdLayout& L, int32_t unit, WideLds& w, uint32_t* bits) {
+  const int lane = threadIdx.x & 63;
+  WsHeader* hdr = reinterpret_cast<WsHeader*>(ws);
+  const int32_t W = (int32_t)((p.K + 31) / 32);
+  const int64_t T = (int64_t)p.R * p.C, P = live_pairs(p, num_pairs), Kl = live_k(p);
+  // the unit's first block; the four are 2 x 2 from there
+  const int32_t rc = kQuad ? p.C : (p.C + 1) / 2;
+  const int32_t ur = unit / rc, uc = unit - ur * rc;
+  const int32_t r0 = 32 * ur, c0 = 32 * uc;
+  if (r0 >= p.M) return;
+  // segment bounds: lane b its block's tile (all four the same tile for kQuad)
+  const int32_t bt = lane & 3;
+  const int32_t tr = kQuad ? ur : 2 * ur + (bt >> 1), tc = kQuad ? uc : 2 * uc + (bt & 1);
+  const bool tile_here = tr < p.R && tc < p.C;
+  const int64_t t = (int64_t)tr * p.C + tc;
+  int64_t s = tile_here ? tile_ptr[t] : 0, e = tile_here ? tile_ptr[t + 1] : 0;
+  if (lane < 4 && tile_here) {
+    if (s < 0 || e < s || e > P) set_status(&hdr->status, GF_STATUS_TILE_PTR_ORDER);
+    if (t == T - 1 && e != P) set_status(&hdr->status, GF_STATUS_TILE_PTR_LAST);
+  }
+  if (s < 0) s = 0;
+  if (e > P) e = P;
+  const int64_t nl = e > s ? e - s : 0;
+  // dL/d(delta-W) of the four blocks, requested together
+  float4 g4[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int32_t lr = r0 + 16 * (b >> 1) + (lane >> 2), lc = c0 + 16 * (b & 1) + ((lane & 3) << 2);
+    const float* gp = grad + (int64_t)min(lr, p.M - 1) * p.N + lc;
+    g4[b] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (lr < p.M) {
+      if (lc + 3 < p.N && ((reinterpret_cast<uintptr_t>(gp) & 15) == 0)) {
+        g4[b] = load4_stream(gp);
+      } else {
+        if (lc < p.N) g4[b].x = load_stream(gp);
+        if (lc + 1 < p.N) g4[b].y = load_stream(gp + 1);
+        if (lc + 2 < p.N) g4[b].z = load_stream(gp + 2);
+        if (lc + 3 < p.N) g4[b].w = load_stream(gp + 3);
+      }
+    }
+  }
+  auto checked_id = [&](int64_t at) -> int32_t {
+    const int64_t g = gids[at];
+    if (g >= 0 && g < Kl) return (int32_t)g;
+    set_status(&hdr->status, g < 0 ? GF_STATUS_IDS_NEGATIVE : GF_STATUS_IDS_RANGE);
+    return -1;
+  };
+  if constexpr (!kQuad) {  // a bit a listed Gaussian, block by block
+    for (int32_t i = lane; i < 4 * W; i += 64) bits[i] = 0u;
+    wave_sync();
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int64_t sb = readlane_i64(s, b), nb = readlane_i64(nl, b);
+      for (int64_t j = lane; j < nb; j += 64) {
+        const int32_t g = checked_id(sb + j);
+        if (g >= 0) atomicOr(bits + (b * W + (g >> 5)), 1u << (g & 31));
+      }
+    }
+  }
+  // the blocks' moments
+  uint32_t fits = 0u;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int32_t br = r0 + 16 * (b >> 1), bc = c0 + 16 * (b & 1);
+    if (br >= p.M || bc >= p.N) continue;
+    *reinterpret_cast<float4*>(w.gt + (lane >> 2) * kWideRow + ((lane & 3) << 2)) = g4[b];
+    if (!poly_grad_fits(g4[b])) continue;
+    fits |= 1u << b;
+    const PolyBlock pb = poly_block(p, row_coords, col_coords, br, bc);
+    if (lane == 0) {
+      *reinterpret_cast<float4*>(&w.block[b][0]) = make_float4(pb.X, pb.Y, pb.sx, pb.sy);
+      *reinterpret_cast<float4*>(&w.block[b][4]) = make_float4(pb.fx, pb.fy, 0.f, 0.f);
+    }
+    poly_moments(p, pb, row_coords, col_coords, br, bc, w.gt, w.pw, w.M[b]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float* const acc_s = reinterpret_cast<float*>(ws + L.acc) + 8 * acc_slot(p, 0, unit & (p.S - 1));
+  bool left = false;
+  // nj listed Gaussians, id_of(j) the j-th (negative: none): a lane each, block after block, or from a
+  // last 32 or fewer two blocks and from a last 16 or fewer all four at once, a lane a (Gaussian, block).
+  auto lanes_of = [](int32_t nj) { return nj > 32 ? 64 : nj > 16 ? 32 : 16; };
+  // The n of them, 64 at a time.  A 64's constants are requested before the atomics of the one before: the memory
+  // counter is in order, and a load behind atomics would wait for them.
+  auto run_list = [&](int32_t n, auto&& id_of) {
+  GaussEval next = zero_eval();
+  int32_t g_next = -1;
+  auto request = [&](int32_t j0) {
+    const int32_t j = lane & (lanes_of(n - j0) - 1);
+    g_next = j0 + j < n ? id_of(j0 + j) : -1;
+    next = zero_eval();
+    if (g_next >= 0) next = load_eval(ev, g_next);
+  };
+  request(0);
+  for (int32_t j0 = 0; j0 < n; j0 += 64) {
+    const int lane = opaque_lane();
+    const int32_t nj = min(64, n - j0), per = lanes_of(nj);
+    const GaussEval my = next;
+    const int32_t g = g_next;
+    float sum[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    bool any = false;
+#pragma unroll 1
+    for (int32_t b0 = 0; b0 < 4; b0 += 64 / per) {
+      const int32_t b = b0 + lane / per;  // the lane's block
+      bool listed = g >= 0 && r0 + 16 * (b >> 1) < p.M && c0 + 16 * (b & 1) < p.N;
+      if (!kQuad && listed) listed = ((bits[b * W + (g >> 5)] >> (g & 31)) & 1u) != 0u;
+      const float4 ba = *reinterpret_cast<const float4*>(&w.block[b][0]), bb = *reinterpret_cast<const float4*>(&w.block[b][4]);
+      const PolyBlock pb{ba.x, ba.y, ba.z, ba.w, bb.x, bb.y, 0, 0};
+      const PolyGauss pg = poly_gauss(pb, my);
+      const bool wide = listed && pg.wide && ((fits >> b) & 1u) != 0u;
+      left = left || (listed && !wide);
+      const uint64_t wb = __builtin_amdgcn_ballot_w64(wide);
+      if (wb == 0ull) continue;
+      float mm[6];
+      if (__builtin_amdgcn_ballot_w64(wide && pg.short_) == wb)
+        poly_six<kPolyShort>(pb, pg, my, w.M[b], mm);
+      else
+        poly_six<kPolyDeg>(pb, pg, my, w.M[b], mm);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) sum[k] += wide ? mm[k] : 0.0f;
+      any = any || wide;
+    }
+    uint64_t taken = __builtin_amdgcn_ballot_w64(any);
+    for (int32_t o = per; o < 64; o <<= 1) {  // the Gaussian's other blocks
+#pragma unroll
+      for (int k = 0; k < 6; ++k) sum[k] += __shfl_xor(sum[k], o, 64);
+      taken |= taken >> o;
+    }
+    if (j0 + 64 < n) request(j0 + 64);
+    // six moments a lane -> eight lanes a Gaussian, half the wave's Gaussians at a time
+    const int32_t to = lane < per && ((taken >> lane) & 1ull) != 0ull ? g : -1;
+    float* ex = w.gt;
+    for (int hf = 0; 32 * hf < nj; ++hf) {
+      if ((lane >> 5) == hf) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) ex[7 * (lane & 31) + k] = sum[k];
+        ex[7 * (lane & 31) + 6] = __int_as_float(to);
+      }
+      wave_sync();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int gi = 8 * i + (lane >> 3), k = lane & 7;
+        const float v = ex[7 * gi + min(k, 5)];
+        const int32_t go = __float_as_int(ex[7 * gi + 6]);
+        if (go >= 0 && k < 6) unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)go + (uint32_t)k), v);
+      }
+      wave_sync();
+    }
+  }
+  };
+  if constexpr (kQuad) {
+    const int64_t sb = readlane_i64(s, 0), nb = readlane_i64(nl, 0);
+    if (nb > 0) run_list((int32_t)min(nb, (int64_t)INT32_MAX), [&](int32_t j) { return checked_id(sb + j); });
+  } else {
+    for (int32_t w0 = 0; w0 < W; w0 += 64) {
+      const int32_t wd = w0 + lane;
+      const uint32_t m = wd < W ? bits[wd] | bits[W + wd] | bits[2 * W + wd] | bits[3 * W + wd] : 0u;
+      const int32_t cnt = __popc(m), inc = dpp_scan_i32(cnt);
+      const int32_t tot = __builtin_amdgcn_readlane(inc, 63);
+      for (int32_t base = 0; base < tot; base += kWideKeys) {
+        uint32_t mm = m;
+        int32_t pos = inc - cnt;
+        while (mm != 0u && pos < base + kWideKeys) {
+          const int32_t bit = __builtin_ctz(mm);
+          mm &= mm - 1u;
+          if (pos >= base) w.keys[pos - base] = (wd << 5) + bit;
+          ++pos;
+        }
+        wave_sync();
+        const int32_t nwin = min(kWideKeys, tot - base);
+        run_list(nwin, [&](int32_t j) { return w.keys[j]; });
+        wave_sync();
+      }
+    }
+  }
+  if (__builtin_amdgcn_ballot_w64(left) != 0ull && lane == 0) atomicOr(&hdr->heavy, 1u);
+}
+
+// Batched wide fields hold the listed-Gaussian bits of up to this many Gaussians.
+constexpr int64_t kWideBatchMaxK = 2048;
+
+// Units of k_bwd_wide, a wave each: 32x32 tiles, or 2x2 tiles of 16x16.
+__host__ __device__ inline int64_t wide_units(const Problem& p) {
+  return p.tile_out == 32 ? (int64_t)p.R * p.C : (int64_t)((p.R + 1) / 2) * ((p.C + 1) / 2);
+}
+// LDS of the listed-Gaussian bits of four waves.
+inline size_t wide_bits_bytes(const Problem& p) {
+  return p.tile_out == 32 ? 0 : sizeof(uint32_t) * (kTileThreads / 64) * 4 * (size_t)((p.K + 31) / 32);
+}
+
+template <bool kQuad>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_bwd_wide(
+    Problem p, const float* __restrict__ grad, const float* __restrict__ row_coords,
+    const float* __restrict__ col_coords, const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr,
+    const int64_t* __restrict__ gids, int64_t num_pairs, uint8_t* ws, BwdLayout L) {
+  __shared__ __align__(16) WideLds lds[kTileThreads / 64];
+  extern __shared__ uint32_t wide_bits[];
+  const int64_t unit = (int64_t)blockIdx.x * (kTileThreads / 64) + wave_id();
+  if (unit >= wide_units(p)) return;
+  bwd_wide_body<kQuad>(p, grad, row_coords, col_coords, ev, tile_ptr, gids, num_pairs, ws, L, (int32_t)unit,
+                       lds[wave_id()], wide_bits + wave_id() * 4 * ((p.K + 31) / 32));
+}
+
+// The rest of a wide field, as k_bwd16's dense form.
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_bwd_rest(
+    Problem p, const float* __restrict__ grad, const float* __restrict__ row_coords,
+    const float* __restrict__ col_coords, const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr,
+    const int64_t* __restrict__ gids, int64_t num_pairs, uint8_t* ws, BwdLayout L) {
+  if (reinterpret_cast<const WsHeader*>(ws)->heavy == 0u) return;
+  bwd16_body<int64_t, int64_t, true, false, true, true, false, true>(p, grad, row_coords, col_coords, nullptr, nullptr,
+                                                                     ev, tile_ptr, gids, num_pairs, ws, L,
+                                                                     sub_tile(p, blockIdx.x, wave_id()));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -3744,6 +4105,7 @@ __device__ __forceinline__ void finish_body(
     const float4* __restrict__ fwd_cov = nullptr, const float2* __restrict__ fwd_lfac = nullptr,
     int32_t ostride = 0, float gscale = 1.0f) {
   float* acc = reinterpret_cast<float*>(ws + L.acc);
+  if (idx == 0) reinterpret_cast<WsHeader*>(ws)->heavy = 0u;  // k_bwd_wide's flag
   const int64_t g = idx / p.S;
   const int32_t st = (int32_t)(idx & (p.S - 1));
   float m[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -4036,8 +4398,9 @@ struct BatchLayer {
   float* d_mu;
   float* d_chol_raw;
   float* d_amp;
-  int64_t tile_block0, emit_block0, finish_block0, render_block0;
+  int64_t tile_block0, emit_block0, finish_block0, render_block0, wide_block0;
   int32_t pair_render;  // rendered by tile pairs (render map); else tile by tile (tile map)
+  int32_t wide;         // in the wide map: reduced by k_bwd_wide_batch where its pairs make it a wide field
   float grad_scale;     // the backward's moments are multiplied by it (merged layers: delta_scale)
   MergedOut mo;         // merged consumer (mo.merged NULL: none)
 };
@@ -4049,7 +4412,7 @@ struct BatchHeader {
   int64_t n;
   int64_t tile_blocks, emit_blocks, finish_blocks, render_blocks;
   int64_t layers_off, tile_map_off, emit_map_off, finish_map_off, render_map_off, grad_table_off, readback_off,
-      total;
+      wide_map_off, total;
 };
 
 struct BatchReadback {
@@ -4060,8 +4423,9 @@ struct BatchReadback {
   double pad2;
 };
 
+// (the wide map comes last: the other regions' places do not depend on it)
 BatchHeader batch_header(int64_t n, int64_t tile_blocks, int64_t emit_blocks, int64_t finish_blocks,
-                         int64_t render_blocks) {
+                         int64_t render_blocks, int64_t wide_blocks = 0) {
   BatchHeader h{};
   h.n = n;
   h.tile_blocks = tile_blocks;
@@ -4075,7 +4439,8 @@ BatchHeader batch_header(int64_t n, int64_t tile_blocks, int64_t emit_blocks, in
   h.render_map_off = (int64_t)align256(h.finish_map_off + sizeof(int32_t) * finish_blocks);
   h.grad_table_off = (int64_t)align256(h.render_map_off + sizeof(int32_t) * render_blocks);
   h.readback_off = (int64_t)align256(h.grad_table_off + sizeof(void*) * n);
-  h.total = (int64_t)align256(h.readback_off + sizeof(BatchReadback) * n);
+  h.wide_map_off = (int64_t)align256(h.readback_off + sizeof(BatchReadback) * n);
+  h.total = (int64_t)align256(h.wide_map_off + sizeof(int32_t) * wide_blocks);
   return h;
 }
 
@@ -4121,7 +4486,8 @@ __device__ inline BatchLayer batch_layer(const uint8_t* plan, int64_t map_off, i
   *block0_sel = which == 0   ? ly.tile_block0
                 : which == 1 ? ly.emit_block0
                 : which == 2 ? ly.finish_block0
-                             : ly.render_block0;
+                : which == 3 ? ly.render_block0
+                             : ly.wide_block0;
   if (index) *index = l;
   return global_layer(ly);
 }
@@ -4187,7 +4553,7 @@ __global__ __launch_bounds__(kTileThreads) void k_render16x2_batch(const uint8_t
 // Eight waves per SIMD: the batch's dense-tile body fits 64 VGPRs without spilling, and the
 // eighth wave hides more of each tile's load chain (cfg4: 397 -> 383 us).
 template <bool kMaskClamp>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bwd16_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bwd16_batch(const uint8_t* __restrict__ plan, int32_t wide_launched) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   int32_t l;
@@ -4197,11 +4563,49 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
   const BwdLayout L = ly.bl;
   const int64_t T = (int64_t)p.R * p.C;
   const int64_t P = ly.tile_ptr[T];  // pairs beyond the id capacity were never emitted
+  if (wide_launched && ly.wide && wide_field(p, min(P, ly.capacity), kWideBatchMinBlocks)) return;  // k_bwd_wide_batch's
   const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
   bwd16_body<int64_t, int64_t, true, kMaskClamp, true, true>(p, grad, ly.row_coords, ly.col_coords, ly.mu, ly.chol_raw,
                                reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
                                ly.tile_ptr, ly.ids, P < ly.capacity ? P : ly.capacity, ly.bws, L,
                                sub_tile(p, (int64_t)blk - b0, wave_id()));
+}
+
+// The wide fields of a batch (over the wide map), and what they leave (over the tile map): k_bwd_wide and k_bwd_rest.
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_bwd_wide_batch(const uint8_t* __restrict__ plan) {
+  const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
+  int64_t b0;
+  int32_t l;
+  const BatchLayer ly = batch_layer(plan, h->wide_map_off, &b0, 4, blockIdx.x, &l);
+  const Problem p = ly.p;
+  const int64_t P = min(ly.tile_ptr[(int64_t)p.R * p.C], ly.capacity);
+  if (!wide_field(p, P, kWideBatchMinBlocks)) return;
+  __shared__ __align__(16) WideLds lds[kTileThreads / 64];
+  __shared__ uint32_t bits[kTileThreads / 64][4 * kWideBatchMaxK / 32];
+  const int64_t unit = ((int64_t)blockIdx.x - b0) * (kTileThreads / 64) + wave_id();
+  if (unit >= wide_units(p)) return;
+  const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
+  const GaussEval* ev = reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval);
+  if (p.tile_out == 32)
+    bwd_wide_body<true>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
+                        lds[wave_id()], bits[wave_id()]);
+  else
+    bwd_wide_body<false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
+                         lds[wave_id()], bits[wave_id()]);
+}
+
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_bwd_rest_batch(const uint8_t* __restrict__ plan) {
+  const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
+  int64_t b0;
+  int32_t l;
+  const BatchLayer ly = batch_layer(plan, h->tile_map_off, &b0, 0, blockIdx.x, &l);
+  if (!ly.wide || reinterpret_cast<const WsHeader*>(ly.bws)->heavy == 0u) return;
+  const Problem p = ly.p;
+  const int64_t P = min(ly.tile_ptr[(int64_t)p.R * p.C], ly.capacity);
+  const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
+  bwd16_body<int64_t, int64_t, true, false, true, true, false, true>(
+      p, grad, ly.row_coords, ly.col_coords, ly.mu, ly.chol_raw, reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
+      ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, sub_tile(p, (int64_t)blockIdx.x - b0, wave_id()));
 }
 
 // dL/d(delta) pointers of layers base .. base + count - 1 (count <= kPtrChunk), passed by value.
@@ -4333,6 +4737,19 @@ void launch_bwd(const Problem& p, dim3 grid, hipStream_t st, const float* grad, 
   const int32_t xh = heavy_list ? heavy_grid(p, num_pairs) : 0;
   const TP* tp = reinterpret_cast<const TP*>(tile_ptr);
   const GI* gi = reinterpret_cast<const GI*>(gids);
+  if constexpr (std::is_same<TP, int64_t>::value && std::is_same<GI, int64_t>::value) {
+    if (ev && dense && wide_field(p, num_pairs)) {
+      Problem q = p;
+      q.heavy = 0;
+      auto wide = p.tile_out == 32 ? k_bwd_wide<true> : k_bwd_wide<false>;
+      const unsigned blocks = (unsigned)((wide_units(p) + kTileThreads / 64 - 1) / (kTileThreads / 64));
+      hipLaunchKernelGGL(wide, dim3(blocks), dim3(kTileThreads), wide_bits_bytes(p), st, q, grad, rc, cc, ev, tp, gi,
+                         num_pairs, ws, L);
+      hipLaunchKernelGGL(k_bwd_rest, dim3((unsigned)quad_grid(p)), dim3(kTileThreads), 0, st, q, grad, rc, cc, ev, tp,
+                         gi, num_pairs, ws, L);
+      return;
+    }
+  }
   if (quad_tiles(p)) {
     if (p.mask_clamp && dense)
       launch_bwd16<TP, GI, true, true>(p, xh, st, grad, rc, cc, mu, raw, ev, tp, gi, num_pairs, ws, L, heavy_list,
@@ -5082,8 +5499,8 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
   const size_t n = (size_t)n_layers;
   BatchHeader h{};
   std::vector<BatchLayer> ls(n);
-  int64_t tile_blocks = 0, emit_blocks = 0, finish_blocks = 0, render_blocks = 0;
-  bool backward_buffers = true, grads_set = true, tile_render = false;
+  int64_t tile_blocks = 0, emit_blocks = 0, finish_blocks = 0, render_blocks = 0, wide_blocks = 0;
+  bool backward_buffers = true, grads_set = true, tile_render = false, wide_pairs = false;
   for (size_t i = 0; i < n; ++i) {
     const gf_layer& in = layers[i];
     BatchLayer& ly = ls[i];
@@ -5146,7 +5563,17 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
     ly.emit_block0 = emit_blocks;
     ly.finish_block0 = finish_blocks;
     ly.render_block0 = render_blocks;
+    ly.wide_block0 = wide_blocks;
     tile_blocks += quad_grid(ly.p);
+    // Whether a layer may become a wide field, at every k <= kc (the map and its grid must not change with k or
+    // the id capacity); whether its pairs make it one, the kernels see.  The launch is left out while no layer's id
+    // capacity has room for a wide field's pairs.
+    ly.wide = quad_tiles(ly.p) && !ly.p.mask_clamp && kc >= 1 && kc <= kWideBatchMaxK &&
+              tile_blocks16(ly.p) >= kWideBatchMinBlocks;
+    if (ly.wide) {
+      wide_blocks += (wide_units(ly.p) + kTileThreads / 64 - 1) / (kTileThreads / 64);
+      wide_pairs = wide_pairs || wide_field(ly.p, in.ids_capacity, kWideBatchMinBlocks);
+    }
     // Tile pairs for 16x16 layers on the mask path at the capacity, hence at every 1 <= k <= kc
     // (each condition of the mask path bounds K from above; the grids must not change with k).
     // The others render tile by tile over the tile map: layers past the masks' K, and layers
@@ -5164,9 +5591,9 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
     if (ly.p.W == 0 || pc.W == 0) emit_blocks += (kc + per_emit_block - 1) / per_emit_block;  // emission path
     finish_blocks += (kc * ly.p.S + kTileThreads - 1) / kTileThreads;
   }
-  if (tile_blocks >= INT32_MAX || emit_blocks >= INT32_MAX || render_blocks >= INT32_MAX)
+  if (tile_blocks >= INT32_MAX || emit_blocks >= INT32_MAX || render_blocks >= INT32_MAX || wide_blocks >= INT32_MAX)
     return set_err(GF_E_INVALID_ARGUMENT, "batch too large for one launch");
-  h = batch_header(n_layers, tile_blocks, emit_blocks, finish_blocks, render_blocks);
+  h = batch_header(n_layers, tile_blocks, emit_blocks, finish_blocks, render_blocks, wide_blocks);
   const size_t need = (size_t)h.total;
   info->n_layers = n_layers;
   info->mask_clamp = (cfg->has_clamp_quad && cfg->clamp_quad < 80.0) ? 1 : 0;
@@ -5177,7 +5604,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
   info->finish_blocks = finish_blocks;
   info->render_blocks = render_blocks;
   info->tile_render = tile_render ? 1 : 0;
-  info->reserved = 0;
+  info->wide_blocks = wide_pairs ? (int32_t)wide_blocks : 0;
   info->plan_bytes = need;
   if (!plan) return GF_OK;  // size query
   if (plan_bytes < need) return set_err(GF_E_WORKSPACE, "batch plan needs %zu bytes, got %zu", need, plan_bytes);
@@ -5188,6 +5615,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
   int32_t* em = reinterpret_cast<int32_t*>(host.data() + h.emit_map_off);
   int32_t* fm = reinterpret_cast<int32_t*>(host.data() + h.finish_map_off);
   int32_t* rmap = reinterpret_cast<int32_t*>(host.data() + h.render_map_off);
+  int32_t* wmap = reinterpret_cast<int32_t*>(host.data() + h.wide_map_off);
   const float** gt = reinterpret_cast<const float**>(host.data() + h.grad_table_off);
   for (size_t i = 0; i < n; ++i) gt[i] = layers[i].grad_delta;
   for (size_t i = 0; i < n; ++i) {
@@ -5199,6 +5627,8 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
     for (int64_t b = ls[i].emit_block0; b < ee; ++b) em[b] = (int32_t)i;
     for (int64_t b = ls[i].finish_block0; b < fe; ++b) fm[b] = (int32_t)i;
     for (int64_t b = ls[i].render_block0; b < re; ++b) rmap[b] = (int32_t)i;
+    const int64_t we = i + 1 < n ? ls[i + 1].wide_block0 : wide_blocks;
+    for (int64_t b = ls[i].wide_block0; b < we; ++b) wmap[b] = (int32_t)i;
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   GF_HIP_CHECK(hipMemcpyAsync(plan, host.data(), need, hipMemcpyHostToDevice, st));
@@ -5283,10 +5713,17 @@ int gf_batch_backward(const void* plan, const gf_batch_info* info, uint32_t phas
   const uint8_t* pl = reinterpret_cast<const uint8_t*>(plan);
   if (phases & GF_PHASE_REDUCE) {
     if (info->mask_clamp)
-      hipLaunchKernelGGL(k_bwd16_batch<true>, dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl);
+      hipLaunchKernelGGL(k_bwd16_batch<true>, dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl, 0);
     else
-      hipLaunchKernelGGL(k_bwd16_batch<false>, dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl);
+      hipLaunchKernelGGL(k_bwd16_batch<false>, dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl,
+                         info->wide_blocks > 0 ? 1 : 0);
     GF_LAUNCH_CHECK("k_bwd16_batch");
+    if (info->wide_blocks > 0 && !info->mask_clamp) {
+      hipLaunchKernelGGL(k_bwd_wide_batch, dim3((unsigned)info->wide_blocks), dim3(kTileThreads), 0, st, pl);
+      GF_LAUNCH_CHECK("k_bwd_wide_batch");
+      hipLaunchKernelGGL(k_bwd_rest_batch, dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl);
+      GF_LAUNCH_CHECK("k_bwd_rest_batch");
+    }
   }
   if ((phases & GF_PHASE_FINISH) && info->finish_blocks > 0) {
     hipLaunchKernelGGL(k_finish_batch, dim3((unsigned)info->finish_blocks), dim3(kTileThreads), 0, st, pl);

@@ -388,7 +388,8 @@ typedef struct gf_batch_info {
   int64_t render_blocks;         /* workgroups of the tile-pair render: 4 pairs of 16x16 tiles each */
   int32_t tile_render;           /* 1: some layer renders tile by tile (32x32 tiles, or a k capacity
                                     past the masks), a second launch over the tile map */
-  int32_t reserved;
+  int32_t wide_blocks;           /* workgroups of the wide-Gaussian reduction (0: no layer's id capacity
+                                    has room for a wide field's pairs) */
 } gf_batch_info;
 
 /*
@@ -411,7 +412,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
  * when every layer is on the mask path). */
 int gf_batch_forward(const void* plan, const gf_batch_info* info, uint32_t phases, void* stream);
 
-/* gf_backward of every layer (with its pair constants): two launches. */
+/* gf_backward of every layer (with its pair constants): two launches, or four with info->wide_blocks. */
 int gf_batch_backward(const void* plan, const gf_batch_info* info, uint32_t phases, void* stream);
 
 /*

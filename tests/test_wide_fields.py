@@ -118,3 +118,85 @@ def test_wide_gaussians_infinite_amplitude(device):
     q = p.to(device)
     delta, _, _ = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, 32, 32, 3.0, False, 80.0)
     assert torch.isposinf(delta).all()
+
+
+# The wide-field backward takes fields of 2048 blocks or more (256 in a batch) whose Gaussians span 192 blocks
+# or more on average: 16x16 and 32x32 tiles, ragged edges, Gaussians left to the element-wise kernel (narrow ones,
+# and those of a block with an infinite dL/d(delta-W)), several times 64 listed, K past a bit row of 1024.
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Nf,K,tile,kind", [
+    (800, 810, 70, 16, "init"), (790, 820, 70, 32, "init"), (800, 810, 150, 16, "mixed"), (800, 810, 150, 32, "mixed"),
+    (730, 800, 1100, 16, "init"), (800, 805, 200, 32, "normalize")])
+def test_wide_field_backward(M, Nf, K, tile, kind, device):
+    from guass_amd.cuda_field import ext
+    from guass_amd.ops import FieldBatchPlan
+    from oracle import field_oracle as fo
+
+    p = _mixed(M, Nf, K, 11) if kind == "mixed" else init_problem(M, Nf, K, 11, sigma=0.35 if K > 1000 else None)
+    norm = kind == "normalize"
+    r = fo.gaussian_field_fwd_bwd_fp64(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, tile, tile, 3.0,
+                                       norm, 80.0)
+    pairs = int(r[1][-1]) * (4 if tile == 32 else 1)
+    assert pairs >= 192 * K and int(r[1][-1]) >= 24 * (r[1].numel() - 1)  # the rule the kernels go by
+    q = p.to(device)
+    args = (tile, tile, 3.0, norm, 80.0)
+    delta, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    field_close(delta, r[0])
+    plain = ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tp, ids, *args)
+    for _ in range(2):  # the accumulators and the flag are clear again in between
+        got = ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tp, ids, *args,
+                                          forward_workspace=ws)
+        for name, a, b, c in zip(("d_mu", "d_chol_raw", "d_amp"), got, r[3:], plain):
+            grad_close(a, b, name, rtol=1e-5)
+            grad_close(c, b, name, rtol=1e-5)
+    layers = [p.to(device), init_problem(320, 330, 40, 12).to(device)]
+    layers[1].grad = torch.randn(320 * 330, generator=torch.Generator().manual_seed(1)).to(device)
+    batch = FieldBatchPlan(layers, device, capacities=[int(r[1][-1]), 400 * 40], tile_out=tile, tile_in=tile, normalize=norm)
+    assert batch.info.wide_blocks > 0
+    for _ in range(2):
+        batch.forward()
+        batch.backward()
+    torch.cuda.synchronize()
+    assert batch.status() == [0, 0]
+    for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), (batch.plans[0].d_mu, batch.plans[0].d_chol_raw, batch.plans[0].d_amp),
+                          r[3:]):
+        grad_close(a, b, f"batch {name}", rtol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [16, 32])
+def test_wide_field_backward_infinite_gradient(tile, device):
+    """One infinite dL/d(delta-W): the Gaussians over it get non-finite gradients as from the element-wise
+    kernels, the others finite ones."""
+    from guass_amd.cuda_field import ext
+
+    p = init_problem(800, 810, 300, 13, sigma=0.2)
+    p.grad[5 * 810 + 7] = float("inf")
+    q = p.to(device)
+    args = (tile, tile, 3.0, False, 80.0)
+    _, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    a, b = (ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tp, ids, *args,
+                                        forward_workspace=w) for w in (ws, None))
+    listed = ids[tp[0]:tp[1]]
+    assert listed.numel() >= 24
+    for x, y in zip(a, b):
+        fin = torch.isfinite(y).all(dim=-1)
+        assert torch.equal(torch.isfinite(x).all(dim=-1), fin)
+        assert not fin[listed].any() and int((~fin).sum()) == listed.numel()
+
+
+@pytest.mark.gpu
+def test_wide_field_backward_checks_saved_state(device):
+    from guass_amd.cuda_field import ext
+
+    p = init_problem(800, 810, 70, 14)
+    q = p.to(device)
+    args = (16, 16, 3.0, False, 80.0)
+    _, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    for edit, msg in ((lambda t, i: i.__setitem__(100, 70), "out-of-range"), (lambda t, i: i.__setitem__(100, -1), "non-negative"),
+                      (lambda t, i: t.__setitem__(9, 0), "monotonic")):
+        t, i = tp.clone(), ids.clone()
+        edit(t, i)
+        with pytest.raises(RuntimeError, match=msg):
+            ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, t, i, *args,
+                                        forward_workspace=ws)
