@@ -1098,7 +1098,8 @@ __device__ inline int32_t prep_store(const Problem& p, const PrepLoad& in, const
 // WsHeader::part entry each.
 static_assert(1024 / 64 <= 16, "a part entry per preparation workgroup");
 
-template <bool kCoef, bool kSplit>
+// kParts (one thread per Gaussian): prep_store's parts (the emission path leaves the constants to k_emit).
+template <bool kCoef, bool kSplit, int kParts = 3>
 __global__ __launch_bounds__(kTilesThreads) void k_prep(Problem p, const float* __restrict__ mu,
                                                         const float* __restrict__ chol_raw,
                                                         const float* __restrict__ amp, uint8_t* ws,
@@ -1127,7 +1128,7 @@ __global__ __launch_bounds__(kTilesThreads) void k_prep(Problem p, const float* 
     const int64_t g = (int64_t)blockIdx.x * kTilesThreads + threadIdx.x;
     if (g < K) {
       const PrepLoad in = prep_load(mu, chol_raw, g);
-      prep_store(p, in, gf_activate_cholesky(in.r11, in.r21, in.r22), amp, g, ws, L, 3);
+      prep_store(p, in, gf_activate_cholesky(in.r11, in.r21, in.r22), amp, g, ws, L, kParts);
     }
     return;
   }
@@ -1165,40 +1166,42 @@ __global__ __launch_bounds__(kTilesThreads) void k_prep(Problem p, const float* 
   }
 }
 
-__global__ __launch_bounds__(kTilesThreads) void k_bin_tiles(Problem p, int64_t* __restrict__ tile_ptr,
-                                                             int64_t* __restrict__ num_pairs, uint8_t* ws,
-                                                             FwdLayout L, const float* __restrict__ chol_raw,
-                                                             const float* __restrict__ amp) {
+// kMasks == false (emission path: R workgroups, a tile row each): tile_ptr alone, with the tiles' fill counters cleared.
+template <bool kMasks, int kThreads>
+__global__ __launch_bounds__(kThreads) void k_bin_tiles(Problem p, int64_t* __restrict__ tile_ptr,
+                                                        int64_t* __restrict__ num_pairs, uint8_t* ws, FwdLayout L,
+                                                        const float* __restrict__ chol_raw,
+                                                        const float* __restrict__ amp) {
   __shared__ int32_t diff[kLdsDiffWords];  // tile-row workgroups: the row's column differences
   const int64_t K = live_k(p);
   const int32_t R = p.R, C = p.C, W = p.W;
   // every mask word is written, those of Gaussians past K as zero (in capacity mode a workspace
   // keeps the words of an earlier, larger K)
-  const int64_t Kw = 32 * (int64_t)W;
+  const int64_t Kw = kMasks ? 32 * (int64_t)W : K;
   const int32_t b = (int32_t)blockIdx.x;
-  const bool is_row = b < R;
+  const bool is_row = !kMasks || b < R;
   const int32_t line = is_row ? b : b - R;
   const int lane = threadIdx.x & 63;
   const int4* __restrict__ rect = reinterpret_cast<const int4*>(ws + L.rect);
   uint32_t* out = reinterpret_cast<uint32_t*>(ws + (is_row ? L.rowmask : L.colmask)) + (int64_t)line * W;
   if (is_row)
-    for (int32_t i = threadIdx.x; i <= C; i += kTilesThreads) diff[i] = 0;
+    for (int32_t i = threadIdx.x; i <= C; i += kThreads) diff[i] = 0;
   __syncthreads();
   int64_t before = 0, pairs = 0;
   int32_t span = 0;  // the most tiles of one rectangle (row workgroups; the last one reports it)
   // The rectangles are loaded kBinPrefetch rounds at a time, so that the rounds do not each wait
   // for their own load (4 rounds at cfg3).
   constexpr int kBinPrefetch = 8;
-  for (int64_t gb = threadIdx.x & ~63; gb < Kw; gb += kBinPrefetch * kTilesThreads) {  // wave-uniform
+  for (int64_t gb = threadIdx.x & ~63; gb < Kw; gb += kBinPrefetch * kThreads) {  // wave-uniform
     int4 rr[kBinPrefetch];
 #pragma unroll
     for (int i = 0; i < kBinPrefetch; ++i) {
-      const int64_t g = gb + (int64_t)i * kTilesThreads + lane;
+      const int64_t g = gb + (int64_t)i * kThreads + lane;
       rr[i] = g < K ? rect[g] : make_int4(0, -1, 0, -1);
     }
 #pragma unroll
     for (int i = 0; i < kBinPrefetch; ++i) {
-      const int64_t g0 = gb + (int64_t)i * kTilesThreads;
+      const int64_t g0 = gb + (int64_t)i * kThreads;
       if (g0 >= Kw) break;
       const int64_t g = g0 + lane;
       bool covers = false;
@@ -1218,6 +1221,7 @@ __global__ __launch_bounds__(kTilesThreads) void k_bin_tiles(Problem p, int64_t*
           covers = r.z <= line && line <= r.w;
         }
       }
+      if constexpr (!kMasks) continue;
       const uint64_t bits = __builtin_amdgcn_ballot_w64(covers);
       const int64_t w0 = g0 >> 5;  // even: words w0, w0 + 1 hold Gaussians g0 .. g0 + 63
       if (lane == 0) out[w0] = (uint32_t)bits;
@@ -1229,7 +1233,7 @@ __global__ __launch_bounds__(kTilesThreads) void k_bin_tiles(Problem p, int64_t*
     // column workgroups finish before the row workgroups' scans)
     const float4* cv = reinterpret_cast<const float4*>(ws + L.cov);
     const float2* lf = reinterpret_cast<const float2*>(ws + L.lfac);
-    for (int64_t g = line + (int64_t)C * threadIdx.x; g < K; g += (int64_t)C * kTilesThreads) {
+    for (int64_t g = line + (int64_t)C * threadIdx.x; g < K; g += (int64_t)C * kThreads) {
       const float4 c4 = cv[g];
       const float2 l = lf[g];
       GfCov c;
@@ -1245,7 +1249,7 @@ __global__ __launch_bounds__(kTilesThreads) void k_bin_tiles(Problem p, int64_t*
   // with D, E the exclusive prefixes of diff[c] and c*diff[c]: one scan of two sums, with
   // rowbase and the pair total as plain sums beside it.  Thread t owns columns
   // [t*per, t*per + per).
-  constexpr int kWaves = kTilesThreads / 64;
+  constexpr int kWaves = kThreads / 64;
   __shared__ int64_t wsum[4][kWaves];
   __shared__ int32_t wspan[kWaves];
   const int wid = threadIdx.x >> 6;
@@ -1253,7 +1257,7 @@ __global__ __launch_bounds__(kTilesThreads) void k_bin_tiles(Problem p, int64_t*
     for (int off = 32; off > 0; off >>= 1) span = max(span, __shfl_xor(span, off));
     if (lane == 0) wspan[wid] = span;
   }
-  const int32_t per = (C + kTilesThreads - 1) / kTilesThreads;
+  const int32_t per = (C + kThreads - 1) / kThreads;
   const int32_t cb = (int32_t)threadIdx.x * per, ce = min(cb + per, C);
   int64_t d = 0, e = 0;
   for (int32_t c = cb; c < ce; ++c) {
@@ -1285,9 +1289,10 @@ __global__ __launch_bounds__(kTilesThreads) void k_bin_tiles(Problem p, int64_t*
   int32_t* heavy_list = reinterpret_cast<int32_t*>(ws + L.fill);
   for (int32_t c = cb; c < ce; ++c) {
     tp[c] = rowbase + (int64_t)c * D - E;
+    if constexpr (!kMasks) heavy_list[(int64_t)line * C + c] = 0;  // the fill counters
     D += diff[c];  // the count of tile (line, c)
     E += (int64_t)c * diff[c];
-    if (p.heavy > 0 && D > p.heavy)
+    if (kMasks && p.heavy > 0 && D > p.heavy)
       heavy_list[atomicAdd(&reinterpret_cast<WsHeader*>(ws)->heavy, 1u)] = line * C + c;
   }
   if (line == R - 1 && threadIdx.x == 0) {
@@ -4944,6 +4949,13 @@ int gf_forward_bin_info(const gf_field_config* cfg, int64_t out_features, int64_
 // force_tiles: bin the tiles with k_bin_tiles (tile_ptr and the chain-rule maps stored here) also
 // where the render would bin them itself (tiles_in_render).  kdev: capacity mode (k is the capacity,
 // the live K is *kdev; see Problem::kdev).
+// Emission path (more Gaussians or words than masks hold): a preparation over the chip and a workgroup per tile row,
+// where one workgroup of k_bin takes all Gaussians through one CU.  Both by call, 16x16 tiles: 2560x5120 K = 16384
+// 116 -> 12 us (370 -> 12 where nearly all tiles are covered), 320x320 K = 16384 60 -> 11, 64x64 K = 9000 40 -> 12,
+// 1280x1280 K = 32768 118 -> 15, 8192x8192 K = 65536 1253 -> 41; every row workgroup reads every rectangle, and still
+// 262144x16 K = 20000 (16384 rows of one tile) 3478 -> 430.  k_bin keeps K = 0 and the grids whose row of column
+// differences does not fit in LDS.
+constexpr int kBinRowsThreads = 1024;
 static int forward_bin(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,
                        const float* mu, const float* chol_raw, const float* amp, int64_t* tile_ptr,
                        int64_t* num_pairs_dev, gf_bin_info* info, void* workspace, size_t workspace_bytes,
@@ -4974,8 +4986,16 @@ static int forward_bin(const gf_field_config* cfg, int64_t out_features, int64_t
     if (in_render) parts = nbp;
     p.heavy = heavy_threshold(p);
     if (!in_render)
-      hipLaunchKernelGGL(k_bin_tiles, dim3(lines), dim3(kTilesThreads), 0, st, p, tile_ptr, num_pairs_dev, ws, L,
-                         chol_raw, amp);
+      hipLaunchKernelGGL((k_bin_tiles<true, kTilesThreads>), dim3(lines), dim3(kTilesThreads), 0, st, p, tile_ptr,
+                         num_pairs_dev, ws, L, chol_raw, amp);
+  } else if (k > 0 && bin_counts_in_lds(p.C, k)) {
+    uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
+    const unsigned nbp = (unsigned)((k + kTilesThreads - 1) / kTilesThreads);
+    hipLaunchKernelGGL((k_prep<false, false, 1>), dim3(nbp), dim3(kTilesThreads), 0, st, p, mu, chol_raw, nullptr, ws, L,
+                       num_pairs_dev);
+    GF_LAUNCH_CHECK("k_prep");
+    hipLaunchKernelGGL((k_bin_tiles<false, kBinRowsThreads>), dim3((unsigned)p.R), dim3(kBinRowsThreads), 0, st, p,
+                       tile_ptr, num_pairs_dev, ws, L, nullptr, nullptr);
   } else {
     hipLaunchKernelGGL(k_bin, dim3(1), dim3(kBinThreads), 0, st, p, mu, chol_raw, tile_ptr,
                        num_pairs_dev, reinterpret_cast<uint8_t*>(workspace), L);
