@@ -13,8 +13,9 @@
 //   row per workgroup (the K rectangles tested against the row once, a barrier, the row's
 //   Gaussians listed in LDS in id order, each wave's two tiles taken from that list), and
 //   k_prep also stores the chain-rule maps.  Up to 256 Gaussians each tile's wave bins itself.
-// Emission path, three kernels:
-//   k_bin      one workgroup per field: rectangles, the pair total, per-tile Gaussian counts
+// Emission path, four kernels:
+//   k_prep, k_bin_tiles as above without the constants and the masks, over the tile rows alone;
+//   k_bin      in their place for no Gaussians and for very wide grids, one workgroup per field: rectangles, the pair total, per-tile Gaussian counts
 //              from row-wise difference arrays and their scan -> tile_ptr; every scan runs in
 //              LDS (DPP wave scans) and global memory is only written, coalesced.  (The
 //              batched form, k_bin_batch, one workgroup per field, also builds the masks.)
@@ -27,6 +28,9 @@
 //              tile's segment, per-Gaussian constants loaded one Gaussian per lane and broadcast
 //              with readlane, 4 pixels per lane with per-row terms hoisted.
 //   (k_render_any handles other tile shapes.)
+// Wide Gaussians (nearly constant over a 16x16 block) go through the block's polynomial instead of
+// element by element ("Wide Gaussians" below): in k_render16, k_render16x2_rows, k_render16_batch
+// and, for the backward of fields made of them, k_bwd_wide (+ k_bwd_rest for what is not wide).
 // Backward (reference backward.cu:541-716), two kernels:
 //   k_bwd16    one wave per 16x16 tile: lanes are (Gaussian slot, tile row); each lane sums
 //              16 pixels of its row for its Gaussian into six moments, 16-lane DPP row sums
@@ -1652,6 +1656,19 @@ constexpr int kPolyMore = 8;  // and a further 64's, whose sums join the first's
 constexpr float kPolyMaxQ = 24.0f;     // (farther ones, whose reach would say little, go element by element)
 constexpr float kPolyMaxAmp = 1e30f;  // amplitudes past this (infinite ones) go element by element
 
+// The tile renders look for wide Gaussians where the mean rectangle covers kPolyBlocks blocks or more (half a wide
+// one's) and, as far as the binning before the render tells, none is kPolySpread times the mean (many small and few huge
+// ones: the search costs more than it finds, 1280x5120 K = 4096 on 32x32 tiles with heavy-tailed log-scales 136 -> 147
+// us).  Their kernel is launched only where the id capacity has room for that: it holds 61-65 vector registers instead of
+// 51 and takes sparse fields 5-10% longer (1280x5120 K = 2048 on 32x32 tiles, 3 a tile: 15.8 -> 17.5 us).
+constexpr int64_t kPolyBlocks = 64, kPolySpread = 16;
+__host__ __device__ inline bool poly_pairs(const Problem& p, int64_t pairs) {
+  return (p.tile_out == 32 && p.tile_in == 32 ? 4 : 1) * pairs >= kPolyBlocks * p.K;
+}
+__device__ inline bool poly_field(const Problem& p, const WsHeader* hdr) {
+  return poly_pairs(p, hdr->pairs) && hdr->max_span * p.K <= kPolySpread * hdr->pairs;
+}
+
 struct PolyBlock {
   float X, Y;    // the block's middle
   float sx, sy;  // scales (powers of two)
@@ -1780,7 +1797,7 @@ __device__ __forceinline__ void poly_sum_add(PolySum& ps, const PolyGauss& o, fl
 // The polynomial of the sums at the lane's elements: row lane / 4, columns 4 (lane % 4) .. + 3, whose offsets
 // xi (row) and eta (columns) are given.  lds: 128 floats of the wave's.
 __device__ __forceinline__ void poly_eval(const PolySum& ps, float xi, const float (&eta)[4], float* lds, float (&out)[4]) {
-  const int lane = threadIdx.x & 63;
+  const int lane = opaque_lane();
   const bool hb0 = (lane & 1) != 0, hb1 = (lane & 2) != 0;
   // each register over its rows' lanes by recursive halving (as the backward's moments): lane bits
   // 3, 2, 1 pick registers (in units of four places) 4 b1 + 2 b2 + b3 in even lanes, 8 + 2 b2 + b3 in odd ones
@@ -1925,9 +1942,11 @@ __shared__ float4 r16_wevals[kTileThreads / 64][128];
 // took 20.1 us).
 constexpr int kRowsThreads = 512;
 __shared__ float4 r16_rows_wevals[kRowsThreads / 64][128];
+// and its wide Gaussians of each of the pair's tiles, by place in the row list
+__shared__ uint32_t r16_rows_wide[kRowsThreads / 64][2 * 32];
 
-constexpr int32_t kWideKey = 1 << 30;  // a key whose Gaussian the block's polynomial holds
-
+// kPoly: wide Gaussians go through their block's polynomial.
+template <bool kPoly>
 __device__ __forceinline__ void render16_body(
     const Problem& p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr, int64_t* ids,
@@ -1949,26 +1968,30 @@ __device__ __forceinline__ void render16_body(
   const bool write_ids = st.quad == 0 && q == 0;  // one wave of a tile writes its ids
   const int32_t pr = st.r0 + (lane >> 2), pc = st.c0 + ((lane & 3) << 2);
   // coordinates first: they do not depend on the tile's segment
-  const float x = row_coords[min(pr, p.M - 1)];
   // The lane's four columns as y0 and offsets from it: z of column i is z0 + wc (y_i - y0), one
   // FMA, with y_i - y0 exact for neighbouring coordinates.
-  float y0, yd[4];
-  {
-    float y[4];
-    if (pc + 3 < p.N && ((reinterpret_cast<uintptr_t>(col_coords + pc) & 15) == 0)) {
-      const float4 v = *reinterpret_cast<const float4*>(col_coords + pc);
+  float x, y[4], y0, yd[4];
+  auto load_coords = [&](int ln) {
+    const int32_t row = st.r0 + (ln >> 2), col = st.c0 + ((ln & 3) << 2);
+    x = row_coords[min(row, p.M - 1)];
+    if (col + 3 < p.N && ((reinterpret_cast<uintptr_t>(col_coords + col) & 15) == 0)) {
+      const float4 v = *reinterpret_cast<const float4*>(col_coords + col);
       y[0] = v.x;
       y[1] = v.y;
       y[2] = v.z;
       y[3] = v.w;
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = col_coords[min(pc + i, p.N - 1)];
+      for (int i = 0; i < 4; ++i) y[i] = col_coords[min(col + i, p.N - 1)];
     }
+  };
+  // (apart from their loads, which the wave does not wait for before its masks)
+  auto offsets = [&]() {
     y0 = y[0];
 #pragma unroll
     for (int i = 0; i < 4; ++i) yd[i] = y[i] - y0;
-  }
+  };
+  load_coords(lane);
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   // With clamp_quad >= 80 (or none) the clamp only floors positive-definite bases below e^-40:
   // the third loop of run_chunk leaves them at their value, a difference below e^-40 |amp| per
@@ -2014,13 +2037,10 @@ __device__ __forceinline__ void render16_body(
   // Gaussians.
   auto& wevals = r16_wevals;
   float4* ew = wevals[wid];
-  // (si: the lane's place among the chunk's Gaussians, negative for none)
-  auto run_chunk = [&](const GaussEval& my, int nj, int si) {
+  auto run_chunk = [&](const GaussEval& my, int nj) {
     // two arrays of 64 float4 (conflict-free writes, broadcast reads)
-    if (si >= 0) {
-      ew[si] = make_float4(my.mu0, my.mu1, my.wa, my.wb);
-      ew[64 + si] = make_float4(my.wc, my.w, __int_as_float(my.gid), my.gen);
-    }
+    ew[lane] = make_float4(my.mu0, my.mu1, my.wa, my.wb);
+    ew[64 + lane] = make_float4(my.wc, my.w, __int_as_float(my.gid), my.gen);
     wave_sync();
     auto at = [&](int j) {
       const float4 a = ew[j], b = ew[64 + j];
@@ -2035,8 +2055,14 @@ __device__ __forceinline__ void render16_body(
       u.gen = b.w;
       return u;
     };
-    if (__builtin_amdgcn_ballot_w64(si >= 0 && my.gen != 0.0f) == 0) {
-      if (floor_free)
+    if (__builtin_amdgcn_ballot_w64(lane < nj && my.gen != 0.0f) == 0) {
+      // Four at a time, their LDS reads together, where the chunk is long (1280x5120 K = 4096 clustered, 32x32 tiles:
+      // 33 -> 30 us; chunks of two or three lose 1 us of 16 to it, and the polynomials need its registers).
+      if (!kPoly && floor_free && nj >= 8)
+#pragma clang loop unroll_count(4)
+        for (int j = 0; j < nj; ++j) accumulate_free(at(j));
+      else if (floor_free)
+#pragma clang loop unroll(disable)
         for (int j = 0; j < nj; ++j) accumulate_free(at(j));
       else
         for (int j = 0; j < nj; ++j) accumulate(at(j), std::false_type{});
@@ -2120,6 +2146,7 @@ __device__ __forceinline__ void render16_body(
     const uint32_t* rm = rowmask + (int64_t)tr * p.W;
     const uint32_t* cm = colmask + (int64_t)tc * p.W;
     int32_t* keys = wkeys[wid];
+    const bool polys = kPoly && F == 1 && floor_free && count >= kPolyMin && (rects || poly_field(p, hdr));
     int64_t done = 0;
     for (int32_t w0 = 0; w0 < p.W; w0 += 64) {
       const int32_t w = w0 + lane;
@@ -2138,19 +2165,21 @@ __device__ __forceinline__ void render16_body(
           ++pos;
         }
         wave_sync();
-        const int32_t nwin = min(kWaveSortKeys, tot - base);
+        int32_t nwin = min(kWaveSortKeys, tot - base);
+        done += nwin;
         if (write_ids) {
           for (int32_t j = lane; j < nwin; j += 64) {
-            const int64_t slot = done + j;
+            const int64_t slot = done - nwin + j;
             if (slot < room) ids[s + slot] = keys[j];
           }
         }
-        // The window's wide Gaussians as one polynomial, 64 at a time where enough of them are; they are
-        // marked in their keys and left out below.
-        bool marked = false;
-        if (F == 1 && floor_free && nwin >= kPolyMin) {
+        // The window's wide Gaussians as one polynomial, 64 at a time where enough of them are; their keys leave
+        // the window.
+        if (kPoly && polys && nwin >= kPolyMin) {
           const PolyBlock pb = poly_block(p, row_coords, col_coords, st.r0, st.c0);
           PolySum ps;
+          bool marked = false;
+          int32_t left = 0;  // keys that stay
           for (int32_t j0 = 0; j0 < nwin; j0 += 64) {
             const bool mine = lane < min(64, nwin - j0);
             const int32_t key = mine ? keys[j0 + lane] : 0;
@@ -2159,41 +2188,42 @@ __device__ __forceinline__ void render16_body(
             const PolyGauss g = poly_gauss(pb, my);
             const bool wide = mine && g.wide;
             const int nw = __popcll(__builtin_amdgcn_ballot_w64(wide));
-            if (nw < (marked ? kPolyMore : kPolyMin)) continue;  // wave-uniform
+            const bool add = nw >= (marked ? kPolyMore : kPolyMin);  // wave-uniform
+            const bool stay = mine && !(add && wide);
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(stay);
+            if (stay)  // (at or before its place, which every lane has read)
+              keys[left + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = key;
+            left += __popcll(bal);
+            if (!add) continue;
             if (!marked) {
 #pragma unroll
               for (int i = 0; i < kPolyRegs; ++i) ps.r[i] = 0.0f;
               marked = true;
             }
             poly_sum_add(ps, g, wide ? my.w * g.e0 : 0.0f);
-            if (wide) keys[j0 + lane] = key | kWideKey;
           }
+          nwin = left;
+          wave_sync();
+          const int ln = opaque_lane();
           if (marked) {
             float eta[4], v[4];
+            const int32_t col = st.c0 + ((ln & 3) << 2);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) eta[i] = ldexpf(col_coords[min(pc + i, p.N - 1)] - pb.Y, -pb.ey);
-            poly_eval(ps, ldexpf(x - pb.X, -pb.ex), eta, reinterpret_cast<float*>(ew), v);
+            for (int i = 0; i < 4; ++i) eta[i] = ldexpf(col_coords[min(col + i, p.N - 1)] - pb.Y, -pb.ey);
+            poly_eval(ps, ldexpf(row_coords[min(st.r0 + (ln >> 2), p.M - 1)] - pb.X, -pb.ex), eta,
+                      reinterpret_cast<float*>(ew), v);
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[i] += v[i];
           }
+          load_coords(ln);  // (not kept in registers over the polynomials)
         }
+        offsets();
         for (int32_t j0 = q * cs; j0 < nwin; j0 += F * cs) {
           const int nj = min(cs, nwin - j0);
           GaussEval my = zero_eval();
-          const int32_t key = lane < nj ? keys[j0 + lane] : kWideKey;
-          if (marked) {
-            const bool mine = (key & kWideKey) == 0;
-            const uint64_t bal = __builtin_amdgcn_ballot_w64(mine);
-            if (bal == 0ull) continue;  // wave-uniform
-            if (mine) my = load_eval(ev, key);
-            run_chunk(my, __popcll(bal), mine ? (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u)) : -1);
-          } else {
-            if (lane < nj) my = load_eval(ev, key);
-            run_chunk(my, nj, lane < nj ? lane : -1);
-          }
+          if (lane < nj) my = load_eval(ev, keys[j0 + lane]);
+          run_chunk(my, nj);
         }
-        done += nwin;
         wave_sync();
       }
     }
@@ -2205,6 +2235,7 @@ __device__ __forceinline__ void render16_body(
   } else {
     tile_range(tile_ptr, t, capacity, &s, &n);
   }
+  if (n > 0) offsets();
   if (n > 0 && n <= 64) {
     // Rank sort of the ids (emission order); each lane gathers its Gaussian's constants while
     // the ranks are computed, then they follow their id to lane `rank` (ds_permute).
@@ -2230,7 +2261,7 @@ __device__ __forceinline__ void render16_body(
       if (srt.gid < 0 || srt.gid >= p.K) set_status(&hdr->status, GF_STATUS_COUNT_MISMATCH);
       if (srt.gid != key) ids[s + lane] = srt.gid;  // lanes whose id moved
     }
-    run_chunk(srt, (int)n, lane < n ? lane : -1);
+    run_chunk(srt, (int)n);
   } else if (n > 64) {
     int64_t* seg = ids + s;
     int32_t* keys = wkeys[wid];
@@ -2246,7 +2277,7 @@ __device__ __forceinline__ void render16_body(
           set_status(&hdr->status, GF_STATUS_COUNT_MISMATCH);  // internal mismatch only
         }
       }
-      run_chunk(my, nj, lane < nj ? lane : -1);
+      run_chunk(my, nj);
     }
   }
   if (F > 1) {
@@ -2320,30 +2351,33 @@ __device__ __forceinline__ void render16x2_body(
   const int64_t ta = (int64_t)tr * p.C + tc;
   const int32_t pr = tr * 16 + (lane >> 2);
   const int32_t pc0 = tc * 16 + ((lane & 3) << 2);
-  const float x = row_coords[min(pr, p.M - 1)];
-  float y0[2], yd[2][4];
+  float x, y0[2], yd[2][4];
   // both tiles' columns inside the matrix from a 16-byte aligned base (the same in every lane):
   // every lane's four columns are one aligned float4, without per-lane tests (the row-binned
   // kernel keeps those, as in the stores below)
   const bool cols4 = !kRows && (tc + 2) * 16 <= p.N && (reinterpret_cast<uintptr_t>(col_coords) & 15) == 0;
+  auto load_coords = [&](int ln) {
+    x = row_coords[min(tr * 16 + (ln >> 2), p.M - 1)];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int32_t pc = pc0 + 16 * h;
-    float y[4];
-    if (cols4 || (pc + 3 < p.N && ((reinterpret_cast<uintptr_t>(col_coords + pc) & 15) == 0))) {
-      const float4 v = *reinterpret_cast<const float4*>(col_coords + pc);
-      y[0] = v.x;
-      y[1] = v.y;
-      y[2] = v.z;
-      y[3] = v.w;
-    } else {
+    for (int h = 0; h < 2; ++h) {
+      const int32_t pc = tc * 16 + ((ln & 3) << 2) + 16 * h;
+      float y[4];
+      if (cols4 || (pc + 3 < p.N && ((reinterpret_cast<uintptr_t>(col_coords + pc) & 15) == 0))) {
+        const float4 v = *reinterpret_cast<const float4*>(col_coords + pc);
+        y[0] = v.x;
+        y[1] = v.y;
+        y[2] = v.z;
+        y[3] = v.w;
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = col_coords[min(pc + i, p.N - 1)];
+        for (int i = 0; i < 4; ++i) y[i] = col_coords[min(pc + i, p.N - 1)];
+      }
+      y0[h] = y[0];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) yd[h][i] = y[i] - y[0];
     }
-    y0[h] = y[0];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) yd[h][i] = y[i] - y[0];
-  }
+  };
+  load_coords(lane);
   float acc[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   const bool floor_free = !p.mask_clamp;
   // The two segments are adjacent: [sa, sb) and [sb, se).
@@ -2399,6 +2433,90 @@ __device__ __forceinline__ void render16x2_body(
   auto room_of = [&](int64_t s, int64_t count) {
     return s < 0 ? 0 : capacity - s < count ? (capacity - s > 0 ? capacity - s : 0) : count;
   };
+  uint32_t* wide_bits = kRows ? r16_rows_wide[wid] : nullptr;
+  bool marked = false;
+  if constexpr (kRows) {
+    // The polynomials come before the loop over the row list and leave only their sums in registers (63 in all, as the
+    // occupancy needs): 1280x5120 K = 1024, fresh (70 Gaussians an element), render 98 -> 61 us.  What remains is three
+    // FMAs a coefficient and the 64 lanes' reduction; tiles of fewer than kPolyMin Gaussians pass by.
+    // The tiles' wide Gaussians as a polynomial each, 64 of the tile's at a time through a queue of (id, place in the
+    // row list); they are marked by their place and left out of that tile below.
+    if (floor_free && max(cnt_a, cnt_b) >= kPolyMin) {  // wave-uniform
+      int32_t* queue = reinterpret_cast<int32_t*>(r16_rows_wevals[wid]);
+      wide_bits[lane] = 0u;
+      wave_sync();
+#pragma clang loop unroll(disable)
+      for (int h = 0; h < 2; ++h) {
+        if ((h ? cnt_b : cnt_a) < kPolyMin) continue;
+        const int32_t col = tc + h;
+        const PolyBlock pb = poly_block(p, row_coords, col_coords, tr * 16, col * 16);
+        PolySum ps;
+        int nwide = 0;
+        int32_t j0 = 0, pend = 0;
+        while (true) {
+          const int ln = opaque_lane();
+          while (pend < 64 && j0 < rb.n) {  // wave-uniform
+            const int32_t j = j0 + ln;
+            const int2 e = j < rb.n ? rb.list[j] : make_int2(0, 0x7fff);
+            const bool in = (e.y & 0xffff) <= col && col <= e.y >> 16;
+            const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
+            if (in)
+              queue[pend + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = e.x | (j << 16);
+            pend += __popcll(bal);
+            j0 += 64;
+          }
+          if (pend == 0) break;
+          wave_sync();
+          const int32_t key = ln < pend ? queue[ln] : 0, rest = 64 + ln < pend ? queue[64 + ln] : 0;
+          GaussEval my = zero_eval();
+          if (ln < pend) my = load_eval(ev, key & 0xffff);
+          wave_sync();
+          if (64 + ln < pend) queue[ln] = rest;
+          const PolyGauss g = poly_gauss(pb, my);
+          const bool wide = ln < pend && g.wide;
+          pend = max(pend - 64, 0);
+          const int nw = __popcll(__builtin_amdgcn_ballot_w64(wide));
+          if (nw < (nwide ? kPolyMore : kPolyMin)) continue;  // wave-uniform
+          if (nwide == 0) {
+#pragma unroll
+            for (int i = 0; i < kPolyRegs; ++i) ps.r[i] = 0.0f;
+          }
+          nwide += nw;
+          const uint32_t place = (uint32_t)key >> 16;
+          if (wide) atomicOr(wide_bits + 32 * h + (place >> 5), 1u << (place & 31));
+          poly_sum_add(ps, g, wide ? my.w * g.e0 : 0.0f);
+        }
+        wave_sync();
+        if (nwide == 0) continue;
+        marked = true;
+        const int ln = opaque_lane();
+        float eta[4], v[4];
+        const int32_t pc = col * 16 + ((ln & 3) << 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) eta[i] = ldexpf(col_coords[min(pc + i, p.N - 1)] - pb.Y, -pb.ey);
+        poly_eval(ps, ldexpf(row_coords[min(tr * 16 + (ln >> 2), p.M - 1)] - pb.X, -pb.ex), eta,
+                  reinterpret_cast<float*>(r16_rows_wevals[wid]), v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (h == 0) acc[0][i] = v[i];
+          else acc[1][i] = v[i];
+        }
+      }
+      // (not kept in registers over the polynomials)
+      const int ln = opaque_lane();
+      load_coords(ln);
+      keep0 = false;
+      if (ln < rb.n) {
+        const int2 e = rb.list[ln];
+        const int32_t z = e.y & 0xffff, w = e.y >> 16;
+        const bool ia = z <= tc && tc <= w, ib = has_b && z <= tc + 1 && tc + 1 <= w;
+        keep0 = ia || ib;
+        key0 = e.x | (ia ? kPairInA : 0) | (ib ? kPairInB : 0);
+        if (keep0) pre0 = load_eval(ev, e.x);
+      }
+    }
+  }
   const int64_t room_a = room_of(sa, cnt_a), room_b = room_of(sb, cnt_b);
   if ((sa < 0 || cnt_a < 0 || cnt_b < 0) && lane == 0) set_status(&hdr->status, GF_STATUS_TILE_PTR_ORDER);
   int32_t* keys = r16_wkeys[kRows ? 0 : wid];  // (not used by kRows)
@@ -2409,8 +2527,9 @@ __device__ __forceinline__ void render16x2_body(
   // the active lane of rank j stages Gaussian j (constants, each tile's amplitude, flags: 1 tile
   // A, 2 tile B, 4 indefinite form) and every lane adds its 8 pixels.
   int32_t done_a = 0, done_b = 0;  // ids of each tile so far (< K)
-  auto run_chunk = [&](int32_t kf, bool active, int nj, const GaussEval* given = nullptr) {
-    const bool in_a = active && (kf & kPairInA) != 0, in_b = active && (kf & kPairInB) != 0;
+  // (kRows, j0: the chunk's first place in the row list)
+  auto run_chunk = [&](int32_t kf, bool active, int nj, int32_t j0, const GaussEval* given = nullptr) {
+    bool in_a = active && (kf & kPairInA) != 0, in_b = active && (kf & kPairInB) != 0;
     const uint64_t bal_a = __builtin_amdgcn_ballot_w64(in_a), bal_b = __builtin_amdgcn_ballot_w64(in_b);
     const int32_t id = kf & kPairIdMask;
     if (in_a) {
@@ -2425,6 +2544,16 @@ __device__ __forceinline__ void render16x2_body(
     }
     done_a += __popcll(bal_a);
     done_b += __popcll(bal_b);
+    if constexpr (kRows) {
+      if (marked) {  // wave-uniform
+        const int32_t word = (j0 + lane) >> 5;
+        in_a = in_a && ((wide_bits[word] >> (lane & 31)) & 1u) == 0u;
+        in_b = in_b && ((wide_bits[32 + word] >> (lane & 31)) & 1u) == 0u;
+        active = in_a || in_b;
+        nj = __popcll(__builtin_amdgcn_ballot_w64(active));
+        if (nj == 0) return;
+      }
+    }
     GaussEval my = zero_eval();
     if (active) my = given ? *given : load_eval(ev, id);
     const int32_t fl = (in_a ? 1 : 0) | (in_b ? 2 : 0) | (my.gen != 0.0f ? 4 : 0);
@@ -2510,7 +2639,7 @@ __device__ __forceinline__ void render16x2_body(
     // 64 row Gaussians at a time: those in tile A or B are a chunk, staged in id order
     {
       const uint64_t bal = __builtin_amdgcn_ballot_w64(keep0);
-      if (bal != 0ull) run_chunk(key0, keep0, __popcll(bal), &pre0);  // wave-uniform
+      if (bal != 0ull) run_chunk(key0, keep0, __popcll(bal), 0, &pre0);  // wave-uniform
     }
     for (int32_t j0 = 64; j0 < rb.n; j0 += 64) {
       const int32_t j = j0 + lane;
@@ -2524,7 +2653,7 @@ __device__ __forceinline__ void render16x2_body(
         kf = e.x | (ia ? kPairInA : 0) | (ib ? kPairInB : 0);
       }
       const uint64_t bal = __builtin_amdgcn_ballot_w64(keep);
-      if (bal != 0ull) run_chunk(kf, keep, __popcll(bal));  // wave-uniform
+      if (bal != 0ull) run_chunk(kf, keep, __popcll(bal), j0);  // wave-uniform
     }
   }
   const uint32_t* rm = kRows ? nullptr : rowmask + (int64_t)tr * p.W;
@@ -2556,7 +2685,7 @@ __device__ __forceinline__ void render16x2_body(
       const int32_t nwin = min(kWaveSortKeys, tot_u - base);
       for (int32_t j0 = 0; j0 < nwin; j0 += 64) {
         const int nj = min(64, nwin - j0);
-        run_chunk(lane < nj ? keys[j0 + lane] : 0, lane < nj, nj);
+        run_chunk(lane < nj ? keys[j0 + lane] : 0, lane < nj, nj, j0);
       }
       wave_sync();
     }
@@ -2712,7 +2841,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_render16x2_rows(
 }
 
 // Single 16x16 fields on the mask path with heavy-tile workgroups: the first workgroups take one
-// listed heavy tile each (four waves, as k_render16<true>), the rest a pair of horizontally
+// listed heavy tile each (four waves, as k_render16<true, false>), the rest a pair of horizontally
 // adjacent tiles a wave (R x ceil(C / 2) pairs, four a workgroup, as k_render16x2), leaving a
 // heavy member of the pair to its own workgroup.
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_render16x2_heavy(
@@ -2729,7 +2858,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
   }
   if (b < nh) {  // the workgroup's four waves share one listed tile
     const int64_t t = heavy_list[b];
-    render16_body(p, row_coords, col_coords, ev, tile_ptr, ids, capacity, delta, ws, rowmask, colmask,
+    render16_body<false>(p, row_coords, col_coords, ev, tile_ptr, ids, capacity, delta, ws, rowmask, colmask,
                   tile16(p, t < 0 || t >= T ? T : t), nullptr, nullptr, wave_id(), kTileThreads / 64);
     return;
   }
@@ -2747,7 +2876,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
                          tc, nullptr, MergedOut{nullptr, nullptr, 1.0f}, skip);
 }
 
-template <bool kHeavy>
+template <bool kHeavy, bool kPoly>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_render16(
     Problem p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr, int64_t* ids,
@@ -2763,7 +2892,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
     it.q = 0;
     it.F = 1;
   }
-  render16_body(p, row_coords, col_coords, ev, tile_ptr, ids, capacity, delta, ws, rowmask, colmask, it.st,
+  render16_body<kPoly>(p, row_coords, col_coords, ev, tile_ptr, ids, capacity, delta, ws, rowmask, colmask, it.st,
                 rects, tile_ptr_out, it.q, it.F);
 }
 
@@ -3420,16 +3549,20 @@ struct WideLds {            // a wave's
   int32_t keys[kWideKeys];
 };
 
-// Lists of kPolyMin Gaussians or more a tile on average, each over kWideBlocks blocks or more (a side of fourteen
-// blocks: a sigma of about 35 elements, poly_gauss's reach), on the masks' K.
-constexpr int64_t kWideBlocks = 192;
+// Lists of kPolyMin Gaussians or more a tile on average, on the masks' K, each over kWideBlocks blocks or more on average:
+// a sigma of about 60 elements, as 35 elements' (192 blocks) is poly_gauss's reach but a heavy-tailed field of 407 blocks
+// a Gaussian is half narrow pairs (1280x5120 K = 4096, Student-t log-scales: 377 us by moments, 316 by tiles; 32x32
+// tiles 953 against 827).  A batch takes the reach itself: its layers are of one kind, and one launch pays for all of
+// them (28 fresh layers of K = 256: 77 us of tiles and 91 of moments at kWideBlocks, 28 and 104 here).
+constexpr int64_t kWideBlocks = 480, kWideBatchBlocks = 192;
 // Single fields of fewer blocks leave most SIMDs without one of these longer waves: 320x320 (400 blocks), K = 32 took
 // 12.8 us against 8.5 for a block a wave.  In a batch the other layers fill them.
 constexpr int64_t kWideMinBlocks = 2048, kWideBatchMinBlocks = 256;
-__host__ __device__ inline bool wide_field(const Problem& p, int64_t pairs, int64_t min_blocks = kWideMinBlocks) {
+__host__ __device__ inline bool wide_field(const Problem& p, int64_t pairs, int64_t min_blocks = kWideMinBlocks,
+                                            int64_t mean_blocks = kWideBlocks) {
   const int64_t q = p.tile_out == 32 && p.tile_in == 32 ? 4 : 1;
   return ((p.tile_out == 16 && p.tile_in == 16) || q == 4) && !p.mask_clamp && p.K >= 1 && p.K <= kMaskMaxK &&
-         q * p.R * p.C >= min_blocks && pairs >= kPolyMin * (int64_t)p.R * p.C && q * pairs >= kWideBlocks * p.K;
+         q * p.R * p.C >= min_blocks && pairs >= kPolyMin * (int64_t)p.R * p.C && q * pairs >= mean_blocks * p.K;
 }
 
 template <bool kQuad>
@@ -4245,9 +4378,12 @@ __global__ __launch_bounds__(256) void k_selftest_softplus(unsigned long long* o
 // such layers from 526 to 366 us; 320x320 with K = 32 from 16.5 to 8.7 us.  With
 // more slots than blocks the finish loses what the reduction gains (28 trained layers of K = 1024:
 // 84.6 -> 81.9 us against 5.2 -> 7.5 us at 1.25 slots a block).
+// Above kStripesFewK Gaussians the finish loses what the reduction gains even below that (1280x1280 K = 1024 on 32x32
+// tiles, trained: 10.2 -> 9.9 against 2.6 -> 3.5 us).
+constexpr int64_t kStripesFewK = 512;
 int32_t backward_stripes(int64_t K, int64_t T, int64_t blocks) {
   int32_t S = T >= 16384 ? 32 : (T >= 8192 ? 8 : (T >= 2048 ? 4 : 1));
-  while (K > 0 && S < kMaxStripes && 2 * S * K <= blocks) S *= 2;
+  while (K > 0 && K <= kStripesFewK && S < kMaxStripes && 2 * S * K <= blocks) S *= 2;
   return S;
 }
 
@@ -4520,6 +4656,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_batch(const uint8_t* __re
 
 // Layers rendered tile by tile (BatchLayer::pair_render == 0: 32x32 tiles, or 16x16 tiles whose
 // capacity reaches the emission path), over the tile map; the other layers' blocks return.
+template <bool kPoly>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_render16_batch(const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
@@ -4527,7 +4664,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
   const BatchLayer ly = batch_layer(plan, h->tile_map_off, &b0, 0, blk);
   if (ly.pair_render) return;
   const Problem p = ly.p;
-  render16_body(p, ly.row_coords, ly.col_coords, reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
+  render16_body<kPoly>(p, ly.row_coords, ly.col_coords, reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
                 ly.tile_ptr, ly.ids, ly.capacity, ly.delta, ly.fws,
                 reinterpret_cast<const uint32_t*>(ly.fws + ly.fl.rowmask),
                 reinterpret_cast<const uint32_t*>(ly.fws + ly.fl.colmask),
@@ -4568,7 +4705,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
   const BwdLayout L = ly.bl;
   const int64_t T = (int64_t)p.R * p.C;
   const int64_t P = ly.tile_ptr[T];  // pairs beyond the id capacity were never emitted
-  if (wide_launched && ly.wide && wide_field(p, min(P, ly.capacity), kWideBatchMinBlocks)) return;  // k_bwd_wide_batch's
+  if (wide_launched && ly.wide && wide_field(p, min(P, ly.capacity), kWideBatchMinBlocks, kWideBatchBlocks)) return;  // k_bwd_wide_batch's
   const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
   bwd16_body<int64_t, int64_t, true, kMaskClamp, true, true>(p, grad, ly.row_coords, ly.col_coords, ly.mu, ly.chol_raw,
                                reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
@@ -4584,7 +4721,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5)
   const BatchLayer ly = batch_layer(plan, h->wide_map_off, &b0, 4, blockIdx.x, &l);
   const Problem p = ly.p;
   const int64_t P = min(ly.tile_ptr[(int64_t)p.R * p.C], ly.capacity);
-  if (!wide_field(p, P, kWideBatchMinBlocks)) return;
+  if (!wide_field(p, P, kWideBatchMinBlocks, kWideBatchBlocks)) return;
   __shared__ __align__(16) WideLds lds[kTileThreads / 64];
   __shared__ uint32_t bits[kTileThreads / 64][4 * kWideBatchMaxK / 32];
   const int64_t unit = ((int64_t)blockIdx.x - b0) * (kTileThreads / 64) + wave_id();
@@ -5117,7 +5254,10 @@ static int forward_render(const gf_field_config* cfg, int64_t out_features, int6
       }
       return GF_OK;
     }
-    hipLaunchKernelGGL(xh > 0 ? k_render16<true> : k_render16<false>, dim3((unsigned)(xh + quad_grid(p))),
+    auto render = k_render16<false, false>;
+    if (xh > 0) render = k_render16<true, false>;
+    else if (binned_here && poly_pairs(p, ids_capacity)) render = k_render16<false, true>;
+    hipLaunchKernelGGL(render, dim3((unsigned)(xh + quad_grid(p))),
                        dim3(kTileThreads), 0, st, p, row_coords, col_coords, ev, tile_ptr, gaussian_ids_sorted,
                        ids_capacity, delta, ws, reinterpret_cast<const uint32_t*>(ws + L.rowmask),
                        reinterpret_cast<const uint32_t*>(ws + L.colmask),
@@ -5592,7 +5732,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
               tile_blocks16(ly.p) >= kWideBatchMinBlocks;
     if (ly.wide) {
       wide_blocks += (wide_units(ly.p) + kTileThreads / 64 - 1) / (kTileThreads / 64);
-      wide_pairs = wide_pairs || wide_field(ly.p, in.ids_capacity, kWideBatchMinBlocks);
+      wide_pairs = wide_pairs || wide_field(ly.p, in.ids_capacity, kWideBatchMinBlocks, kWideBatchBlocks);
     }
     // Tile pairs for 16x16 layers on the mask path at the capacity, hence at every 1 <= k <= kc
     // (each condition of the mask path bounds K from above; the grids must not change with k).
@@ -5675,7 +5815,8 @@ int gf_batch_forward(const void* plan, const gf_batch_info* info, uint32_t phase
       GF_LAUNCH_CHECK("k_render16x2_batch");
     }
     if (info->tile_render) {
-      hipLaunchKernelGGL(k_render16_batch, dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl);
+      hipLaunchKernelGGL((info->wide_blocks > 0 ? k_render16_batch<true> : k_render16_batch<false>),
+                         dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl);
       GF_LAUNCH_CHECK("k_render16_batch");
     }
   }
