@@ -4378,12 +4378,12 @@ __global__ __launch_bounds__(256) void k_selftest_softplus(unsigned long long* o
 // such layers from 526 to 366 us; 320x320 with K = 32 from 16.5 to 8.7 us.  With
 // more slots than blocks the finish loses what the reduction gains (28 trained layers of K = 1024:
 // 84.6 -> 81.9 us against 5.2 -> 7.5 us at 1.25 slots a block).
-// Above kStripesFewK Gaussians the finish loses what the reduction gains even below that (1280x1280 K = 1024 on 32x32
-// tiles, trained: 10.2 -> 9.9 against 2.6 -> 3.5 us).
-constexpr int64_t kStripesFewK = 512;
+// Above kStripesFewK Gaussians while 2 S * K is: the finish loses sooner what the reduction gains (1280x1280 K = 1024 on
+// 32x32 tiles, trained: reduction 10.2 -> 9.8 us and finish 2.7 -> 3.5 at a slot per block, 10.0 and 3.2 at half of that).
+constexpr int64_t kStripesFewK = 128;
 int32_t backward_stripes(int64_t K, int64_t T, int64_t blocks) {
   int32_t S = T >= 16384 ? 32 : (T >= 8192 ? 8 : (T >= 2048 ? 4 : 1));
-  while (K > 0 && K <= kStripesFewK && S < kMaxStripes && 2 * S * K <= blocks) S *= 2;
+  while (K > 0 && S < kMaxStripes && (K <= kStripesFewK ? 2 : 4) * S * K <= blocks) S *= 2;
   return S;
 }
 
