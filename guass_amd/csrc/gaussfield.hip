@@ -2331,7 +2331,7 @@ struct RowBin {
   int64_t* tile_ptr_out;     // tile_ptr, written for the wave's tiles (and [T] by tile T - 1's wave)
 };
 
-template <bool kSkipHalves, bool kRows = false>
+template <bool kSkipHalves, bool kRows = false, bool kPoly = false>
 __device__ __forceinline__ void render16x2_body(
     const Problem& p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr, int64_t* __restrict__ ids,
@@ -2433,9 +2433,10 @@ __device__ __forceinline__ void render16x2_body(
   auto room_of = [&](int64_t s, int64_t count) {
     return s < 0 ? 0 : capacity - s < count ? (capacity - s > 0 ? capacity - s : 0) : count;
   };
-  uint32_t* wide_bits = kRows ? r16_rows_wide[wid] : nullptr;
+  uint32_t* wide_bits = nullptr;
+  if constexpr (kRows && kPoly) wide_bits = r16_rows_wide[wid];
   bool marked = false;
-  if constexpr (kRows) {
+  if constexpr (kRows && kPoly) {
     // The polynomials come before the loop over the row list and leave only their sums in registers (63 in all, as the
     // occupancy needs): 1280x5120 K = 1024, fresh (70 Gaussians an element), render 98 -> 61 us.  What remains is three
     // FMAs a coefficient and the 64 lanes' reduction; tiles of fewer than kPolyMin Gaussians pass by.
@@ -2544,7 +2545,7 @@ __device__ __forceinline__ void render16x2_body(
     }
     done_a += __popcll(bal_a);
     done_b += __popcll(bal_b);
-    if constexpr (kRows) {
+    if constexpr (kRows && kPoly) {
       if (marked) {  // wave-uniform
         const int32_t word = (j0 + lane) >> 5;
         in_a = in_a && ((wide_bits[word] >> (lane & 31)) & 1u) == 0u;
@@ -2824,6 +2825,9 @@ __device__ inline RowBin bin_tile_row(const Problem& p, const int4* __restrict__
 // row list at their rank (the mask words' popcounts before its word, then its lane's rank in
 // the word), with their column ranges; after a second barrier each wave renders its pair from
 // the list (render16x2_body<kRows>), which also gives the segment starts in closed form.
+// kPoly: the tiles' wide Gaussians as polynomials, where the id capacity has room for a field of them (poly_pairs;
+// without the search 57 registers, not 63, and trained 1280x1280 K = 1024 8.9 us instead of 9.0).
+template <bool kPoly>
 __global__ __launch_bounds__(kRowsThreads) void k_render16x2_rows(
     Problem p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, int64_t* tile_ptr, int64_t* ids, int64_t capacity,
@@ -2836,7 +2840,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_render16x2_rows(
   const int32_t pc = ((int32_t)blockIdx.x - tr * G) * kWaves + wave_id();  // the wave's pair
   const RowBin rb = bin_tile_row<kRowsThreads>(p, rects, tr, rl, tile_ptr);
   if (pc >= cp) return;  // past the row's last pair (no barrier follows)
-  render16x2_body<false, true>(p, row_coords, col_coords, ev, nullptr, ids, capacity, delta, ws, nullptr, nullptr,
+  render16x2_body<false, true, kPoly>(p, row_coords, col_coords, ev, nullptr, ids, capacity, delta, ws, nullptr, nullptr,
                                tr, 2 * pc, nullptr, MergedOut{nullptr, nullptr, 1.0f}, 0u, rb);
 }
 
@@ -5226,7 +5230,7 @@ static int forward_render(const gf_field_config* cfg, int64_t out_features, int6
   if (quad_render(p)) {
     if (rows_in_render(p)) {
       const int32_t cp = (p.C + 1) / 2, G = (cp + kRowsThreads / 64 - 1) / (kRowsThreads / 64);
-      hipLaunchKernelGGL(k_render16x2_rows, dim3((unsigned)((int64_t)p.R * G)), dim3(kRowsThreads), 0, st, p,
+      hipLaunchKernelGGL((poly_pairs(p, ids_capacity) ? k_render16x2_rows<true> : k_render16x2_rows<false>), dim3((unsigned)((int64_t)p.R * G)), dim3(kRowsThreads), 0, st, p,
                          row_coords, col_coords, ev, tile_ptr, gaussian_ids_sorted, ids_capacity, delta, ws,
                          reinterpret_cast<const int4*>(ws + L.rect));
       GF_LAUNCH_CHECK("k_render16x2_rows");
