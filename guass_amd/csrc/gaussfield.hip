@@ -1779,7 +1779,15 @@ struct PolySum {
   float r[kPolyRegs];
 };
 
-__device__ __forceinline__ void poly_sum_add(PolySum& ps, const PolyGauss& o, float c00) {
+// w: the Gaussian's amplitude; lanes with in == false add nothing.  (Their constants are cleared with their amplitude:
+// a Gaussian that is not wide may have infinite ones, and 0 * inf would reach every element through the sums.)
+__device__ __forceinline__ void poly_sum_add(PolySum& ps, PolyGauss o, bool in, float w) {
+  const float c00 = in ? w * o.e0 : 0.0f;
+  o.L1 = in ? o.L1 : 0.0f;
+  o.L2 = in ? o.L2 : 0.0f;
+  o.Q11x2 = in ? o.Q11x2 : 0.0f;
+  o.Q12 = in ? o.Q12 : 0.0f;
+  o.Q22x2 = in ? o.Q22x2 : 0.0f;
   float q[4], lo = 0.0f;
   poly_coefs<kPolyDeg>(o, c00, [&](int a, int b, const float* cur, const float*, const float*) {
     const int i = a * (kPolyDeg + 1) - a * (a - 1) / 2 + b;  // the coefficient's place in the order
@@ -2200,7 +2208,7 @@ __device__ __forceinline__ void render16_body(
               for (int i = 0; i < kPolyRegs; ++i) ps.r[i] = 0.0f;
               marked = true;
             }
-            poly_sum_add(ps, g, wide ? my.w * g.e0 : 0.0f);
+            poly_sum_add(ps, g, wide, my.w);
           }
           nwin = left;
           wave_sync();
@@ -2486,7 +2494,7 @@ __device__ __forceinline__ void render16x2_body(
           nwide += nw;
           const uint32_t place = (uint32_t)key >> 16;
           if (wide) atomicOr(wide_bits + 32 * h + (place >> 5), 1u << (place & 31));
-          poly_sum_add(ps, g, wide ? my.w * g.e0 : 0.0f);
+          poly_sum_add(ps, g, wide, my.w);
         }
         wave_sync();
         if (nwide == 0) continue;

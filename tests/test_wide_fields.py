@@ -125,6 +125,33 @@ def test_wide_gaussians_infinite_amplitude(device):
     assert torch.isposinf(delta).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", [(0, float("inf")), (1, float("inf")), (1, float("-inf"))])
+@pytest.mark.parametrize("M,Nf,K,tile", [(320, 320, 100, 32), (320, 320, 300, 16)])
+def test_wide_gaussians_infinite_mean(M, Nf, K, tile, where, device):
+    """A Gaussian with an infinite mean among wide ones: its exponent is -inf wherever it is listed, so the field
+    is that of the others (single fields of both renders, and the batch)."""
+    from guass_amd.cuda_field import ext
+    from guass_amd.ops import FieldBatchPlan
+
+    p = init_problem(M, Nf, K, 3, sigma=0.7)
+    p.mu[10, where[0]] = where[1]
+    rest = wl.FieldProblem(p.name, M, Nf, p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp.clone(), p.grad)
+    rest.amp[10] = 0.0
+    rest.mu = p.mu.clone()
+    rest.mu[10] = 0.0
+    args = (tile, tile, 3.0, False, 80.0)
+    q, o = p.to(device), rest.to(device)
+    want = ext.gaussian_field_forward(o.row_coords, o.col_coords, o.mu, o.chol_raw, o.amp, *args)[0].cpu()
+    got, tp, _ = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    pairs = int(tp[-1])
+    assert pairs * (4 if tile == 32 else 1) >= 64 * K  # the rule of the single fields' polynomial kernels
+    field_close(got, want)
+    batch = FieldBatchPlan([q], device, capacities=[pairs], tile_out=tile, tile_in=tile)
+    batch.forward()
+    field_close(batch.plans[0].delta, want)
+
+
 # The wide-field backward takes fields of 2048 blocks or more (256 in a batch) whose Gaussians span 480 blocks
 # or more on average (192 in a batch): 16x16 and 32x32 tiles, ragged edges, Gaussians left to the element-wise kernel (narrow ones,
 # and those of a block with an infinite dL/d(delta-W)), several times 64 listed, K past a bit row of 1024.
