@@ -1671,7 +1671,7 @@ __device__ inline bool poly_field(const Problem& p, const WsHeader* hdr) {
 
 struct PolyBlock {
   float X, Y;    // the block's middle
-  float sx, sy;  // scales (powers of two)
+  float sx, sy;  // scales (powers of two; 0 for a block of one row or column, whose only offset is 0)
   float fx, fy;  // max |xi|, max |eta|
   int ex, ey;    // log2 of the scales
 };
@@ -1692,8 +1692,10 @@ __device__ inline PolyBlock poly_block(const Problem& p, const float* __restrict
   const float xd = row_coords[min(r0 + l16, p.M - 1)] - k.X, yd = col_coords[min(c0 + l16, p.N - 1)] - k.Y;
   const float hx = readlane_f(row16_max(fabsf(xd)), 0), hy = readlane_f(row16_max(fabsf(yd)), 0);  // uniform
   const int ex = __builtin_amdgcn_frexp_expf(hx), ey = __builtin_amdgcn_frexp_expf(hy);
-  k.sx = ldexpf(1.0f, ex);
-  k.sy = ldexpf(1.0f, ey);
+  // (one row: the coefficients of xi's powers would grow with the inverse covariance, which no test bounds, past
+  // the largest number, and meet xi = 0)
+  k.sx = hx == 0.0f ? 0.0f : ldexpf(1.0f, ex);
+  k.sy = hy == 0.0f ? 0.0f : ldexpf(1.0f, ey);
   k.fx = ldexpf(hx, -ex);
   k.fy = ldexpf(hy, -ey);
   k.ex = ex;

@@ -152,6 +152,36 @@ def test_wide_gaussians_infinite_mean(M, Nf, K, tile, where, device):
     field_close(batch.plans[0].delta, want)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Nf,K,backward", [(17, 2000, 96, False), (2000, 17, 96, False), (17, 2000, 300, False),
+                                             (2000, 17, 300, False), (17, 17600, 60, True), (17600, 17, 60, True)])
+def test_wide_gaussians_on_blocks_of_one_row(M, Nf, K, backward, device):
+    """Gaussians as thin as the activation allows (1e-5) across the last block's only row or column: nothing in
+    that block depends on the coefficients of the missing direction, however large."""
+    from guass_amd.cuda_field import ext
+    from oracle import field_oracle as fo
+
+    p = init_problem(M, Nf, K, 4, sigma=0.9)
+    thin = 0 if M == 17 else 1
+    p.mu[:, thin] = 1.0 - 1e-5
+    p.chol_raw[:, 1] = 0.0
+    p.chol_raw[:, 2 * thin] = -25.0
+    p.amp *= 1e5
+    args = (16, 16, 3.0, False, 80.0)
+    r = fo.gaussian_field_fwd_bwd_fp64(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, *args)
+    pairs, T = int(r[1][-1]), r[1].numel() - 1
+    assert pairs >= 64 * K  # the rules of the polynomial kernels
+    q = p.to(device)
+    delta, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    field_close(delta, r[0])
+    if backward:
+        assert pairs >= 480 * K and pairs >= 24 * T and T >= 2048
+        got = ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tp, ids, *args,
+                                          forward_workspace=ws)
+        for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), got, r[3:]):
+            grad_close(a, b, name, rtol=1e-5)
+
+
 # The wide-field backward takes fields of 2048 blocks or more (256 in a batch) whose Gaussians span 480 blocks
 # or more on average (192 in a batch): 16x16 and 32x32 tiles, ragged edges, Gaussians left to the element-wise kernel (narrow ones,
 # and those of a block with an infinite dL/d(delta-W)), several times 64 listed, K past a bit row of 1024.
