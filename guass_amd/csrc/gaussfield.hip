@@ -1632,36 +1632,38 @@ __device__ inline int opaque_lane() {
 // two, |xi|, |eta| <= 1),
 //   e = e0 exp(-(L1 xi + L2 eta + Q11 xi^2 + Q12 xi eta + Q22 eta^2)) = sum_ab c_ab xi^a eta^b,
 //   (a + 1) c_{a+1,b} = -(L1 c_ab + 2 Q11 c_{a-1,b} + Q12 c_{a,b-1}),   c_00 = e0,
-// cut at total degree kPolyDeg.  The render sums the c_ab of a block's wide Gaussians (a lane each)
-// and evaluates one polynomial; the backward takes the block's moments of dL/d(delta-W) against
-// xi^a eta^b once and each Gaussian's six moments from its c_ab and those.  The work per (Gaussian,
-// block) is 45 coefficients of three FMAs instead of 256 exponentials.
+// cut at total degree kPolyDeg in the render, which sums the c_ab of a block's wide Gaussians (a lane each)
+// and evaluates one polynomial: 45 coefficients of three FMAs a (Gaussian, block) instead of 256 exponentials.
+// The backward takes the block's moments of dL/d(delta-W) against xi^a eta^b once and each Gaussian's six moments
+// from its c_ab, up to kPolyDeg or kMomentDeg, and those (of two degrees more, as the second moments meet xi^2 c_ab).
 //
-// What the cut leaves out.  With l = max |L1 xi| + |L2 eta| and k the same bound of the quadratic terms, the terms past
-// degree D of exp(l t + k t^2) bound it (times e0, at a corner of the block): 1e-6 for D = 8 along l + 8 k = 0.85, and
-// growing like (l + 8 k)^(D + 1).  A Gaussian is wide in a block where e0 times that stays below 1e-6, that is where
-// l + 8 k <= kPolyReach e0^(-1 / 9).  A round Gaussian of 36 elements' sigma or more is wide in every block its 3-sigma
-// box meets.  The block's average is a twentieth of the corner's, and against 64 bits the polynomials are closer than
-// summing exponentials (Gaussians of 35-120 elements' sigma: 1.5e-7..2.2e-7 of the norm against 2.2e-7..3.1e-7):
-// 64 lanes' terms add in a tree, and one exponential's argument is rounded instead of 256.
-constexpr int kPolyDeg = 8;
-constexpr float kPolyReach = 0.85f;
-// Where it holds for every Gaussian of the 64, degree 6 does (28 coefficients): 1.5e-6 along l + 8 k = 0.5.
-constexpr int kPolyShort = 6;
-constexpr float kPolyShortReach = 0.5f;
+// What the cut leaves out, relative to the Gaussian's own value at an element.  With l the bound of |L1 xi| + |L2 eta|
+// and k that of the quadratic terms, the series of exp(-(l t + k t^2)) cut at its degree is off at t = 1 by at most
+//   2^-24 (2 + 4 q)   for   l + 8 k <= reach (1 + 2 q)^(1 / (degree + 2)),   q = -ln e0
+// (reached in a corner of the block, by l alone).  That is what an exponential an element costs too: its exponent is
+// rounded there, and far from the mean such values were measured off by 2^-24 5 q.  The error stays with the values
+// of the block itself, however small e0 is; bounded against the amplitude, dL/d(delta-W) in one far block gave
+// gradients off by 7e-4 of themselves where element by element they are by 3e-5.  q <= kPolyMaxQ (in powers of
+// two): farther Gaussians go element by element.
+// A round Gaussian of 66 elements' sigma is wide in every block that its 3-sigma box meets, one of 45 in those of the
+// backward's degree.  Against 64 bits the render of such fields is closer than summing exponentials (60 elements'
+// sigma: 5.7e-8 of the norm against 1.5e-7): 64 lanes' terms add in a tree, and one exponent is rounded for the block.
+constexpr int kPolyDeg = 8, kMomentDeg = 10;
+constexpr float kPolyReach = 0.655f, kMomentReach = 1.05f;
 // Fewer wide Gaussians than this in 64 do not repay the reduction and the evaluation (about 450
 // instructions a block against 24-34 a Gaussian).
 constexpr int kPolyMin = 24;
 constexpr int kPolyMore = 8;  // and a further 64's, whose sums join the first's
-constexpr float kPolyMaxQ = 24.0f;     // (farther ones, whose reach would say little, go element by element)
+constexpr float kPolyMaxQ = 24.0f;
 constexpr float kPolyMaxAmp = 1e30f;  // amplitudes past this (infinite ones) go element by element
 
-// The tile renders look for wide Gaussians where the mean rectangle covers kPolyBlocks blocks or more (half a wide
-// one's) and, as far as the binning before the render tells, none is kPolySpread times the mean (many small and few huge
-// ones: the search costs more than it finds, 1280x5120 K = 4096 on 32x32 tiles with heavy-tailed log-scales 136 -> 147
-// us).  Their kernel is launched only where the id capacity has room for that: it holds 61-65 vector registers instead of
-// 51 and takes sparse fields 5-10% longer (1280x5120 K = 2048 on 32x32 tiles, 3 a tile: 15.8 -> 17.5 us).
-constexpr int64_t kPolyBlocks = 64, kPolySpread = 16;
+// The tile renders look for wide Gaussians where the mean rectangle covers kPolyBlocks blocks or more (fresh layers, 8 in
+// a batch on 32x32 tiles, with the search and without: 640x640 at 349 blocks 47 and 59 us, at 259 64 and 62, 320x320 at
+// 268 21 and 25, at 215 26.2 and 26.5) and, as far as the binning before the render tells, none is kPolySpread times
+// the mean (many small and few huge ones: the search costs more than it finds, 1280x5120 K = 4096 on 32x32 tiles with
+// heavy-tailed log-scales 136 -> 147 us).  Their kernel is launched only where the id capacity has room for that: it
+// holds 61-63 vector registers instead of 51.
+constexpr int64_t kPolyBlocks = 256, kPolySpread = 16;
 __host__ __device__ inline bool poly_pairs(const Problem& p, int64_t pairs) {
   return (p.tile_out == 32 && p.tile_in == 32 ? 4 : 1) * pairs >= kPolyBlocks * p.K;
 }
@@ -1706,8 +1708,8 @@ __device__ inline PolyBlock poly_block(const Problem& p, const float* __restrict
 // A Gaussian's exponent about a block, and whether the polynomial stands for it there.
 struct PolyGauss {
   float L1, L2, Q11x2, Q12, Q22x2, e0;
-  bool wide;   // degree kPolyDeg stands for it
-  bool short_; // so does degree kPolyShort
+  bool wide;    // degree kPolyDeg stands for it
+  bool moment;  // degree kMomentDeg does (the backward's)
 };
 __device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
 #pragma clang fp contract(off)
@@ -1720,11 +1722,12 @@ __device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
   const float lin = (2.0f * ln2) * ((fabsf(la) + fabsf(lb)) * k.fx + fabsf(lc) * k.fy);
   const float h = fabsf(be) * k.fx + fabsf(ga) * k.fy, v = al * k.fx;
   // (comparisons that a NaN fails)
-  const float reach = lin + (8.0f * ln2) * (v * v + h * h);
   const float q = __builtin_fmaf(z0, z0, a0 * a0);
-  o.wide = u.gen == 0.0f && reach <= kPolyReach * __builtin_amdgcn_exp2f(q * (1.0f / (kPolyDeg + 1))) &&
-           q <= kPolyMaxQ && fabsf(u.w) <= kPolyMaxAmp;
-  o.short_ = o.wide && reach <= kPolyShortReach * __builtin_amdgcn_exp2f(q * (1.0f / (kPolyShort + 1)));
+  const float reach = lin + (8.0f * ln2) * (v * v + h * h);
+  const float far = __builtin_amdgcn_logf(__builtin_fmaf(q, 2.0f * ln2, 1.0f));  // log2(1 + 2 q)
+  o.moment = u.gen == 0.0f && reach <= kMomentReach * __builtin_amdgcn_exp2f(far * (1.0f / (kMomentDeg + 2))) &&
+             q <= kPolyMaxQ && fabsf(u.w) <= kPolyMaxAmp;
+  o.wide = o.moment && reach <= kPolyReach * __builtin_amdgcn_exp2f(far * (1.0f / (kPolyDeg + 2)));
   o.L1 = (2.0f * ln2) * (la + lb);
   o.L2 = (2.0f * ln2) * lc;
   o.Q11x2 = (2.0f * ln2) * (al * al + be * be);
@@ -1733,38 +1736,51 @@ __device__ inline PolyGauss poly_gauss(const PolyBlock& k, const GaussEval& u) {
   o.e0 = __builtin_amdgcn_exp2f(-q);
   return o;
 }
+// e0 with its exponent in double: its rounding is the whole block's, where element by element roundings average out
+// (sigma of 75 elements, dL/d(delta-W) in one block: the worst gradient 6e-7 off instead of 1.2e-6; by tiles 2.3e-6).
+__device__ inline float poly_e0(const PolyBlock& k, const GaussEval& u) {
+  constexpr float ln2 = 0.69314718055994530942f;
+  const double dx = (double)k.X - (double)u.mu0, dy = (double)k.Y - (double)u.mu1;
+  const double a = (double)u.wa * dx, z = __builtin_fma((double)u.wc, dy, (double)u.wb * dx);
+  const double qd = __builtin_fma(z, z, a * a);
+  const float q = (float)qd, e = __builtin_amdgcn_exp2f(-q);
+  return __builtin_fmaf(e * ln2, (float)((double)q - qd), e);
+}
 
 // The coefficients c_ab of c00 * e / e0, a + b <= D, a-major: emit(a, b, c_a, c_{a-1}, c_{a-2}), rows indexed by b,
-// is called as c_ab is computed (c_a so far; the rows before are zero past the degree and before the first).
-template <int D, typename Emit>
+// is called as c_ab is computed (c_a so far; the rows before are zero before the first), and for the a + b up to
+// D + X past them.
+template <int D, int X, typename Emit>
 __device__ __forceinline__ void poly_coefs(const PolyGauss& o, float c00, Emit&& emit) {
   float prev[D + 1], prev2[D + 1];
 #pragma unroll
   for (int b = 0; b <= D; ++b) prev[b] = prev2[b] = 0.0f;
 #pragma unroll
-  for (int a = 0; a <= D; ++a) {
+  for (int a = 0; a <= D + X; ++a) {
     float cur[D + 1];
     const float n1 = a > 0 ? o.L1 * (-1.0f / (a > 0 ? a : 1)) : 0.0f, n2 = a > 1 ? o.Q11x2 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
     const float n3 = a > 0 ? o.Q12 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
 #pragma unroll
-    for (int b = 0; b <= D - a; ++b) {
-      float v;
-      if (a == 0) {
-        v = c00;
-        if (b > 0) v = (o.L2 * (-1.0f / (b > 0 ? b : 1))) * cur[b - 1];
-        if (b > 1) v = fmaf(o.Q22x2 * (-1.0f / (b > 0 ? b : 1)), cur[b - 2], v);
-      } else {
-        v = n1 * prev[b];
-        if (a > 1) v = fmaf(n2, prev2[b], v);
-        if (b > 0) v = fmaf(n3, prev[b - 1], v);
+    for (int b = 0; b <= D + X - a; ++b) {
+      if (a + b <= D) {
+        float v;
+        if (a == 0) {
+          v = c00;
+          if (b > 0) v = (o.L2 * (-1.0f / (b > 0 ? b : 1))) * cur[b - 1];
+          if (b > 1) v = fmaf(o.Q22x2 * (-1.0f / (b > 0 ? b : 1)), cur[b - 2], v);
+        } else {
+          v = n1 * prev[b];
+          if (a > 1) v = fmaf(n2, prev2[b], v);
+          if (b > 0) v = fmaf(n3, prev[b - 1], v);
+        }
+        cur[b] = v;
       }
-      cur[b] = v;
       emit(a, b, cur, prev, prev2);
     }
 #pragma unroll
-    for (int b = 0; b <= D - a; ++b) {
-      prev2[b] = prev[b];
-      prev[b] = cur[b];
+    for (int b = 0; b <= D; ++b) {
+      if (a + b <= D + 1) prev2[b] = prev[b];
+      if (a + b <= D) prev[b] = cur[b];
     }
     __builtin_amdgcn_sched_barrier(0);  // a row at a time: the rows ahead would hold registers
   }
@@ -1791,7 +1807,7 @@ __device__ __forceinline__ void poly_sum_add(PolySum& ps, PolyGauss o, bool in, 
   o.Q12 = in ? o.Q12 : 0.0f;
   o.Q22x2 = in ? o.Q22x2 : 0.0f;
   float q[4], lo = 0.0f;
-  poly_coefs<kPolyDeg>(o, c00, [&](int a, int b, const float* cur, const float*, const float*) {
+  poly_coefs<kPolyDeg, 0>(o, c00, [&](int a, int b, const float* cur, const float*, const float*) {
     const int i = a * (kPolyDeg + 1) - a * (a - 1) / 2 + b;  // the coefficient's place in the order
     q[i & 3] = cur[b];
     const bool last = i == kPolyCoefs - 1;  // place 44, the first of its four, in the upper half of a register
@@ -3007,11 +3023,13 @@ __device__ inline void stage_gaussians(const Problem& p, const GIdx* __restrict_
 
 // The backward's side of the polynomial form (poly_coefs).
 //
-// M[a][b] = sum over a block of dL/d(delta-W) xi^a eta^b, a + b <= kPolyDeg, as two products of 16x16 matrices on
+// M[a][b] = sum over a block of dL/d(delta-W) xi^a eta^b, a + b <= kMomentPow, as two products of 16x16 matrices on
 // the matrix cores (fp32): R = G Vy, then M = Vx^T R.  gt: the block's dL/d(delta-W), rows of kWideRow floats; pw:
-// 288 floats for the powers; M: rows of 12.
+// the powers, 32 floats each; M: rows of kMomentRow.
 constexpr int kWideRow = 20;
-constexpr int kPolyM = 12 * (kPolyDeg + 1);
+constexpr int kMomentPow = kMomentDeg + 2;  // the second moments' xi^2 and eta^2 on the last coefficients
+constexpr int kMomentRow = 16;
+static_assert(kMomentPow < kMomentRow, "a row of the moments");
 __device__ __forceinline__ void poly_moments(const Problem& p, const PolyBlock& k, const float* __restrict__ row_coords,
                                              const float* __restrict__ col_coords, int32_t r0, int32_t c0,
                                              const float* gt, float* pw, float* M) {
@@ -3021,13 +3039,13 @@ __device__ __forceinline__ void poly_moments(const Problem& p, const PolyBlock& 
                              : ldexpf(col_coords[min(c0 + l16, p.N - 1)] - k.Y, -k.ey);
     float e = 1.0f;
 #pragma unroll
-    for (int i = 0; i <= kPolyDeg; ++i) {
+    for (int i = 0; i <= kMomentPow; ++i) {
       pw[32 * i + lane] = e;
       e *= v;
     }
   }
   wave_sync();
-  const int e = min(l16, kPolyDeg);  // (lanes past the degree repeat it, and are not stored)
+  const int e = min(l16, kMomentPow);  // (lanes past the degree repeat it, and are not stored)
   const float* px = pw + 32 * e;
   const float* py = px + 16;
   f32x4_t r = {0.f, 0.f, 0.f, 0.f}, m = {0.f, 0.f, 0.f, 0.f};
@@ -3041,7 +3059,7 @@ __device__ __forceinline__ void poly_moments(const Problem& p, const PolyBlock& 
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int a = 4 * grp + i;
-    if (a + l16 <= kPolyDeg) M[12 * a + l16] = m[i];
+    if (a + l16 <= kMomentPow) M[kMomentRow * a + l16] = m[i];
   }
   wave_sync();
 }
@@ -3052,21 +3070,21 @@ __device__ inline bool poly_grad_fits(const float4& g) {
   return __builtin_amdgcn_ballot_w64(!(fabsf(g.x) <= kPolyMaxAmp && fabsf(g.y) <= kPolyMaxAmp &&
                                        fabsf(g.z) <= kPolyMaxAmp && fabsf(g.w) <= kPolyMaxAmp)) == 0ull;
 }
-// The six moments of the lane's Gaussian (about its mean) from the block's: sums of c_ab M[a + i][b + j] for
-// i + j <= 2 within the degree (each M read once, beside the rows it meets), shifted from the block's middle.
+// The six moments of the lane's Gaussian (about its mean) from the block's: sums of c_ab M[a + i][b + j], a + b <= D,
+// for i + j <= 2 (each M read once, beside the rows it meets), shifted from the block's middle.
 template <int D>
 __device__ __forceinline__ void poly_six(const PolyBlock& k, const PolyGauss& o, const GaussEval& u, const float* M,
                                          float (&m)[6]) {
   float s00 = 0.f, s10 = 0.f, s01 = 0.f, s20 = 0.f, s11 = 0.f, s02 = 0.f;
   f32x4_t v;
-  poly_coefs<D>(o, o.e0, [&](int a, int b, const float* cur, const float* prev, const float* prev2) {
-    if ((b & 3) == 0) v = *reinterpret_cast<const f32x4_t*>(M + 12 * a + b);
+  poly_coefs<D, 2>(o, o.e0, [&](int a, int b, const float* cur, const float* prev, const float* prev2) {
+    if ((b & 3) == 0) v = *reinterpret_cast<const f32x4_t*>(M + kMomentRow * a + b);
     const float m_ab = v[b & 3];
-    s00 = fmaf(cur[b], m_ab, s00);
-    if (b > 0) s01 = fmaf(cur[b - 1], m_ab, s01);
-    if (b > 1) s02 = fmaf(cur[b - 2], m_ab, s02);
-    if (a > 0) s10 = fmaf(prev[b], m_ab, s10);
-    if (a > 0 && b > 0) s11 = fmaf(prev[b - 1], m_ab, s11);
+    if (a + b <= D) s00 = fmaf(cur[b], m_ab, s00);
+    if (a <= D && b > 0 && a + b - 1 <= D) s01 = fmaf(cur[b - 1], m_ab, s01);
+    if (a <= D && b > 1) s02 = fmaf(cur[b - 2], m_ab, s02);
+    if (a > 0 && a + b - 1 <= D) s10 = fmaf(prev[b], m_ab, s10);
+    if (a > 0 && a - 1 <= D && b > 0) s11 = fmaf(prev[b - 1], m_ab, s11);
     if (a > 1) s20 = fmaf(prev2[b], m_ab, s20);
   });
   const float dx = k.X - u.mu0, dy = k.Y - u.mu1;
@@ -3239,7 +3257,7 @@ __device__ __forceinline__ void bwd16_body(
         myg = (int32_t)g;
       }
     }
-    const uint64_t skip = kRest && grad_fits ? __builtin_amdgcn_ballot_w64(myg >= 0 && poly_gauss(pb, my).wide) : 0ull;
+    const uint64_t skip = kRest && grad_fits ? __builtin_amdgcn_ballot_w64(myg >= 0 && poly_gauss(pb, my).moment) : 0ull;
     if (kRest && skip != 0ull) {
       // the others to the front, in order
       const bool rest = ((skip >> lane) & 1ull) == 0 && lane < nj;
@@ -3557,20 +3575,23 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
 constexpr int kWideKeys = 256;
 struct WideLds {            // a wave's
   float gt[16 * kWideRow];  // a block's dL/d(delta-W); later the moments on their way out
-  float pw[32 * (kPolyDeg + 1)];
-  float M[4][kPolyM];
+  float M[4][kMomentRow * (kMomentPow + 1)];
   float block[4][8];  // PolyBlock's X, Y, sx, sy, fx, fy
-  int32_t keys[kWideKeys];
+  union {
+    float pw[32 * (kMomentPow + 1)];  // until the moments are there
+    int32_t keys[kWideKeys];
+  };
 };
 
 // Lists of kPolyMin Gaussians or more a tile on average, on the masks' K, each over kWideBlocks blocks or more on average:
-// a sigma of about 60 elements, as 35 elements' (192 blocks) is poly_gauss's reach but a heavy-tailed field of 407 blocks
-// a Gaussian is half narrow pairs (1280x5120 K = 4096, Student-t log-scales: 377 us by moments, 316 by tiles; 32x32
-// tiles 953 against 827).  A batch takes the reach itself: its layers are of one kind, and one launch pays for all of
-// them (28 fresh layers of K = 256: 77 us of tiles and 91 of moments at kWideBlocks, 28 and 104 here).
+// a sigma of about 60 elements, as a heavy-tailed field of 407 blocks a Gaussian is half narrow pairs (1280x5120
+// K = 4096, Student-t log-scales: 377 us by moments, 316 by tiles; 32x32 tiles 953 against 827).  A batch, whose
+// layers are mostly of one kind, goes down to 192 (8 fresh layers of 640x640 on 32x32 tiles, by moments and by tiles:
+// 58 and 76 us at 298 blocks, 66 and 92 at 259, 79 and 87 at 226).
 constexpr int64_t kWideBlocks = 480, kWideBatchBlocks = 192;
 // Single fields of fewer blocks leave most SIMDs without one of these longer waves: 320x320 (400 blocks), K = 32 took
-// 12.8 us against 8.5 for a block a wave.  In a batch the other layers fill them.
+// 12.8 us against 8.5 for a block a wave.  In a batch the other layers fill them (28 of 320x320, K = 64: 38 us by
+// moments, 47 by tiles; 8 of them 26 and 21).
 constexpr int64_t kWideMinBlocks = 2048, kWideBatchMinBlocks = 256;
 __host__ __device__ inline bool wide_field(const Problem& p, int64_t pairs, int64_t min_blocks = kWideMinBlocks,
                                             int64_t mean_blocks = kWideBlocks) {
@@ -3692,16 +3713,17 @@ __device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __r
       if (!kQuad && listed) listed = ((bits[b * W + (g >> 5)] >> (g & 31)) & 1u) != 0u;
       const float4 ba = *reinterpret_cast<const float4*>(&w.block[b][0]), bb = *reinterpret_cast<const float4*>(&w.block[b][4]);
       const PolyBlock pb{ba.x, ba.y, ba.z, ba.w, bb.x, bb.y, 0, 0};
-      const PolyGauss pg = poly_gauss(pb, my);
-      const bool wide = listed && pg.wide && ((fits >> b) & 1u) != 0u;
+      PolyGauss pg = poly_gauss(pb, my);
+      const bool wide = listed && pg.moment && ((fits >> b) & 1u) != 0u;
       left = left || (listed && !wide);
       const uint64_t wb = __builtin_amdgcn_ballot_w64(wide);
       if (wb == 0ull) continue;
+      pg.e0 = poly_e0(pb, my);
       float mm[6];
-      if (__builtin_amdgcn_ballot_w64(wide && pg.short_) == wb)
-        poly_six<kPolyShort>(pb, pg, my, w.M[b], mm);
-      else
+      if (__builtin_amdgcn_ballot_w64(wide && pg.wide) == wb)
         poly_six<kPolyDeg>(pb, pg, my, w.M[b], mm);
+      else
+        poly_six<kMomentDeg>(pb, pg, my, w.M[b], mm);
 #pragma unroll
       for (int k = 0; k < 6; ++k) sum[k] += wide ? mm[k] : 0.0f;
       any = any || wide;
@@ -3775,7 +3797,7 @@ inline size_t wide_bits_bytes(const Problem& p) {
 }
 
 template <bool kQuad>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_bwd_wide(
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_bwd_wide(
     Problem p, const float* __restrict__ grad, const float* __restrict__ row_coords,
     const float* __restrict__ col_coords, const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr,
     const int64_t* __restrict__ gids, int64_t num_pairs, uint8_t* ws, BwdLayout L) {
@@ -4728,7 +4750,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
 }
 
 // The wide fields of a batch (over the wide map), and what they leave (over the tile map): k_bwd_wide and k_bwd_rest.
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_bwd_wide_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_bwd_wide_batch(const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   int32_t l;

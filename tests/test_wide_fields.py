@@ -4,7 +4,10 @@ from __future__ import annotations
 
 import ctypes
 import math
+import re
+from pathlib import Path
 
+import numpy as np
 import pytest
 import torch
 
@@ -38,6 +41,24 @@ def test_backward_workspace_grows_with_k(shape, tile):
     lib, cfg = N.lib(), ctypes.byref(N.make_config(tile, tile, 3.0, False, 80.0))
     need = [lib.gf_backward_workspace_bytes(*shape, k, cfg) for k in range(0, 2200, 7)]
     assert all(a <= b for a, b in zip(need, need[1:]))
+
+
+@pytest.mark.parametrize("deg,reach", [("kPolyDeg", "kPolyReach"), ("kMomentDeg", "kMomentReach")])
+def test_cut_series_keeps_its_bound(deg, reach):
+    """The degrees and reaches of the kernels: the series of exp(-(l t + k t^2)) cut at the degree is within
+    2^-24 (2 + 4 q) of its value at t = 1, over every l and k that the test for wide Gaussians lets pass."""
+    src = (Path(N.__file__).parent / "csrc" / "gaussfield.hip").read_text()
+    D = int(re.search(rf"\b{deg} = (\d+)", src).group(1))
+    R = float(re.search(rf"\b{reach} = ([0-9.]+)f", src).group(1))
+    max_q = float(re.search(r"\bkPolyMaxQ = ([0-9.]+)f", src).group(1)) * math.log(2.0)
+    for q in (0.0, 0.1, 0.5, 1.0, 2.0, 4.5, 9.0, 13.0, max_q):
+        most = R * (1.0 + 2.0 * q) ** (1.0 / (D + 2))
+        l, k = np.meshgrid(np.linspace(-most, most, 301), np.linspace(0.0, most / 8.0, 81), indexing="ij")
+        c = [np.ones_like(l)]
+        for n in range(D):
+            c.append(-(l * c[n] + (2.0 * k * c[n - 1] if n else 0.0)) / (n + 1))
+        err = np.abs(sum(c) * np.exp(l + k) - 1.0) * (np.abs(l) + 8.0 * k <= most)
+        assert err.max() <= 2.0**-24 * (2.0 + 4.0 * q), (q, err.max())
 
 
 @pytest.mark.gpu
@@ -145,7 +166,7 @@ def test_wide_gaussians_infinite_mean(M, Nf, K, tile, where, device):
     want = ext.gaussian_field_forward(o.row_coords, o.col_coords, o.mu, o.chol_raw, o.amp, *args)[0].cpu()
     got, tp, _ = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
     pairs = int(tp[-1])
-    assert pairs * (4 if tile == 32 else 1) >= 64 * K  # the rule of the single fields' polynomial kernels
+    assert pairs * (4 if tile == 32 else 1) >= 256 * K  # the rule of the single fields' polynomial kernels
     field_close(got, want)
     batch = FieldBatchPlan([q], device, capacities=[pairs], tile_out=tile, tile_in=tile)
     batch.forward()
@@ -153,8 +174,8 @@ def test_wide_gaussians_infinite_mean(M, Nf, K, tile, where, device):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,Nf,K,backward", [(17, 2000, 96, False), (2000, 17, 96, False), (17, 2000, 300, False),
-                                             (2000, 17, 300, False), (17, 17600, 60, True), (17600, 17, 60, True)])
+@pytest.mark.parametrize("M,Nf,K,backward", [(17, 6000, 96, False), (6000, 17, 96, False), (17, 6000, 300, False),
+                                             (6000, 17, 300, False), (17, 17600, 60, True), (17600, 17, 60, True)])
 def test_wide_gaussians_on_blocks_of_one_row(M, Nf, K, backward, device):
     """Gaussians as thin as the activation allows (1e-5) across the last block's only row or column: nothing in
     that block depends on the coefficients of the missing direction, however large."""
@@ -170,7 +191,7 @@ def test_wide_gaussians_on_blocks_of_one_row(M, Nf, K, backward, device):
     args = (16, 16, 3.0, False, 80.0)
     r = fo.gaussian_field_fwd_bwd_fp64(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, *args)
     pairs, T = int(r[1][-1]), r[1].numel() - 1
-    assert pairs >= 64 * K  # the rules of the polynomial kernels
+    assert pairs >= 256 * K  # the rules of the polynomial kernels
     q = p.to(device)
     delta, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
     field_close(delta, r[0])
@@ -180,6 +201,114 @@ def test_wide_gaussians_on_blocks_of_one_row(M, Nf, K, backward, device):
                                           forward_workspace=ws)
         for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), got, r[3:]):
             grad_close(a, b, name, rtol=1e-5)
+
+
+def _exponents(p: wl.FieldProblem, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
+    """Each Gaussian's exponent q [K, len(x), len(y)] in float64."""
+    raw, mu = p.chol_raw.double().to(x.device), p.mu.double().to(x.device)
+    l11, l21, l22 = (torch.nn.functional.softplus(raw[:, 0]) + 1e-5, raw[:, 1],
+                     torch.nn.functional.softplus(raw[:, 2]) + 1e-5)
+    u = (x.double()[None] - mu[:, :1]) / l11[:, None]
+    v = ((y.double()[None] - mu[:, 1:])[:, None] - (l21[:, None] * u)[:, :, None]) / l22[:, None, None]
+    return 0.5 * (u.square()[:, :, None] + v.square())
+
+
+def _spread(M: int, Nf: int, K: int, sigma: tuple[float, float], seed: int, around: float | None = None):
+    """K Gaussians of about sigma elements, anywhere or within `around` elements' sigma of the middle."""
+    g = torch.Generator().manual_seed(seed)
+    p = init_problem(M, Nf, K, seed)
+    unit = torch.tensor([2.0 / (M - 1), 2.0 / (Nf - 1)])
+    p.mu = (1.98 * torch.rand(K, 2, generator=g) - 0.99 if around is None
+            else (around * unit * torch.randn(K, 2, generator=g)).clamp(-0.99, 0.99)).contiguous()
+    s = torch.tensor(sigma) * unit * torch.exp(0.1 * torch.randn(K, 2, generator=g))
+    raw = torch.log(torch.expm1(s))
+    p.chol_raw = torch.stack((raw[:, 0], 0.1 * s[:, 1] * torch.randn(K, generator=g), raw[:, 1]), dim=-1).contiguous()
+    p.amp = 1e-3 * (0.5 + torch.rand(K, 1, generator=g))
+    return p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sigma_mult", [3.0, 5.0])
+@pytest.mark.parametrize("sigma", [(36.0, 36.0), (60.0, 60.0), (30.0, 120.0)])
+@pytest.mark.parametrize("M,Nf,K,tile", [(640, 640, 100, 32), (640, 640, 400, 16)])
+def test_wide_gaussians_far_elements(M, Nf, K, tile, sigma, sigma_mult, device):
+    """Positive Gaussians about the middle: every element, also where all n that its tile lists are far away and
+    small, is right to the rounding of its own terms: 2^-24 (8 + 8 q) of each (in first order the covariance's entries,
+    their factor, the offsets, the products and the square are up to 16 roundings of half a unit, in a square; the cut may
+    leave out 2 + 4 q) and 2^-24 2 sqrt(n) of their sum (n roundings of half a unit and of any sign, 7 times their
+    standard deviation)."""
+    from guass_amd.cuda_field import ext
+    from oracle import field_oracle as fo
+
+    p = _spread(M, Nf, K, sigma, 1, around=15.0)
+    args = (tile, tile, sigma_mult, False, 80.0)
+    r = fo.gaussian_field_fwd_bwd_fp64(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, *args)[0]
+    q = p.to(device)
+    delta, tp, ids = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    ref = r.double().view(M, Nf).to(device)
+    err = (delta.double().view(M, Nf) - ref).abs()
+    worst = 0.0
+    for r0 in range(0, M, 64):  # the terms that an element's tile lists
+        x = _exponents(p, q.row_coords[r0:r0 + 64], q.col_coords)
+        # (past the clamp, x = 40, the render leaves exp(-x) where the reference has exp(-40))
+        value = q.amp.double()[:, :, None] * torch.exp(-x)
+        term = value * (8.0 + 8.0 * x) * 2.0**-24 + q.amp.double()[:, :, None] * math.exp(-40.0)
+        for t0 in range(r0, r0 + 64, tile):
+            for t in range(t0 // tile * (Nf // tile), (t0 // tile + 1) * (Nf // tile)):
+                c0 = (t % (Nf // tile)) * tile
+                listed = ids[int(tp[t]):int(tp[t + 1])]
+                e = err[t0:t0 + tile, c0:c0 + tile]
+                if listed.numel() == 0:
+                    assert not bool(e.any())
+                    continue
+                at = (listed, slice(t0 - r0, t0 - r0 + tile), slice(c0, c0 + tile))
+                bound = term[at].sum(0) + 2.0**-23 * math.sqrt(listed.numel()) * value[at].sum(0)
+                worst = max(worst, float((e / bound).max()))
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sigma_mult", [3.0, 5.0])
+@pytest.mark.parametrize("sigma,tile", [((60.0, 60.0), 16), ((60.0, 60.0), 32), ((75.0, 75.0), 32), ((50.0, 200.0), 16)])
+def test_wide_field_backward_of_one_block(sigma, tile, sigma_mult, device):
+    """Positive dL/d(delta-W) in one 16x16 block, or one of its elements: no other block's terms hide an error there,
+    and each Gaussian's gradient (in units of its amplitude and its axes, so that d_amp, a sum of positive terms, sets
+    its scale) is right to the rounding of its exponent in the block, 2^-24 (16 + 32 q) with q the largest over the
+    block: the cut's 2 + 4 q, times 8 for the chain rule's sums of moments."""
+    from guass_amd.cuda_field import ext
+    from oracle import field_oracle as fo
+
+    M = Nf = 1280
+    p = _spread(M, Nf, 256, sigma, 2)
+    args = (tile, tile, sigma_mult, False, 80.0)
+    q = p.to(device)
+    _, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    pairs = int(tp[-1]) * (4 if tile == 32 else 1)
+    assert pairs >= 480 * p.mu.shape[0]  # the rule the kernels go by
+    axes, one = torch.nn.functional.softplus(p.chol_raw[:, ::2]).double(), torch.ones(p.mu.shape[0], dtype=torch.float64)
+    for b0, b1 in ((40, 40), (0, 0), (25, 62)):
+        rows, cols = slice(16 * b0, 16 * b0 + 16), slice(16 * b1, 16 * b1 + 16)
+        t = (16 * b0 // tile) * (Nf // tile) + 16 * b1 // tile
+        listed = ids[int(tp[t]):int(tp[t + 1])].cpu()
+        x = _exponents(p, p.row_coords[rows], p.col_coords[cols]).flatten(1).amax(1)[listed]
+        for only in (None, (15, 15), (0, 15)):
+            block = 0.5 + torch.rand(16, 16, generator=torch.Generator().manual_seed(b0))
+            if only is not None:
+                block = torch.zeros(16, 16)
+                block[only] = 1.0
+            grad = torch.zeros(M, Nf)
+            grad[rows, cols] = block
+            # the block by itself, every Gaussian listed
+            r = fo.gaussian_field_fwd_bwd_fp64(p.row_coords[rows], p.col_coords[cols], p.mu, p.chol_raw, p.amp,
+                                               block.reshape(-1), 16, 16, 1e3, False, 80.0)
+            got = ext.gaussian_field_backward(grad.reshape(-1).to(device), q.row_coords, q.col_coords, q.mu, q.chol_raw,
+                                              q.amp, tp, ids, *args, forward_workspace=ws)
+            a, b = (torch.cat((m.double() * axes, c.double() * torch.stack((one, axes[:, 1], one), -1), d.double() * p.amp), -1)[listed]
+                    for m, c, d in ([v.cpu() for v in got], r[3:]))
+            off = (a - b).norm(dim=-1) / b.norm(dim=-1)
+            near = x <= 40.0  # (beyond, the values leave the numbers' range)
+            worst = float((off / (2.0**-24 * (16.0 + 32.0 * x)))[near].max())
+            assert worst <= 1.0, (b0, b1, only, worst)
 
 
 # The wide-field backward takes fields of 2048 blocks or more (256 in a batch) whose Gaussians span 480 blocks
