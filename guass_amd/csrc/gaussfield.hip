@@ -1661,14 +1661,30 @@ constexpr float kPolyMaxAmp = 1e30f;  // amplitudes past this (infinite ones) go
 // a batch on 32x32 tiles, with the search and without: 640x640 at 349 blocks 47 and 59 us, at 259 64 and 62, 320x320 at
 // 268 21 and 25, at 215 26.2 and 26.5) and, as far as the binning before the render tells, none is kPolySpread times
 // the mean (many small and few huge ones: the search costs more than it finds, 1280x5120 K = 4096 on 32x32 tiles with
-// heavy-tailed log-scales 136 -> 147 us).  Their kernel is launched only where the id capacity has room for that: it
-// holds 61-63 vector registers instead of 51.
+// heavy-tailed log-scales 136 -> 147 us).  The kernels go by the field's own pairs and rectangles (poly_field), so that
+// the same field has the same bits at every id capacity.  Their launch is left out where the id capacity has no room
+// for such a field (poly_room): they hold 61-63 vector registers instead of 51-57 (trained 1280x5120 K = 256 on 32x32
+// tiles 22.9 us with them, 21.6 without).
 constexpr int64_t kPolyBlocks = 256, kPolySpread = 16;
-__host__ __device__ inline bool poly_pairs(const Problem& p, int64_t pairs) {
-  return (p.tile_out == 32 && p.tile_in == 32 ? 4 : 1) * pairs >= kPolyBlocks * p.K;
+__host__ __device__ inline bool poly_pairs(const Problem& p, int64_t K, int64_t pairs) {
+  return pairs >= kPolyBlocks / (p.tile_out == 32 && p.tile_in == 32 ? 4 : 1) * K;
 }
-__device__ inline bool poly_field(const Problem& p, const WsHeader* hdr) {
-  return poly_pairs(p, hdr->pairs) && hdr->max_span * p.K <= kPolySpread * hdr->pairs;
+// (in capacity mode any live K may come)
+bool poly_room(const Problem& p, int64_t ids_capacity) { return poly_pairs(p, p.kdev ? 1 : p.K, ids_capacity); }
+// parts: the tiles are binned in the render, and the preparation's workgroups left their sums (WsHeader::part).
+__device__ inline bool poly_field(const Problem& p, const WsHeader* hdr, bool parts) {
+  const int64_t K = live_k(p);
+  int64_t pairs = hdr->pairs, span = hdr->max_span;
+  if (parts) {
+    const int lane = threadIdx.x & 63;
+    const bool in = lane < (p.K + 63) / 64;
+    const int32_t n = in ? hdr->part[lane & 15][0] : 0;
+    int32_t most = in ? hdr->part[lane & 15][1] : 0;
+    for (int off = 8; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off));
+    pairs = __builtin_amdgcn_readlane(dpp_scan_i32(n), 63);
+    span = __builtin_amdgcn_readlane(most, 0);
+  }
+  return poly_pairs(p, K, pairs) && span * K <= kPolySpread * pairs;
 }
 
 struct PolyBlock {
@@ -2172,7 +2188,7 @@ __device__ __forceinline__ void render16_body(
     const uint32_t* rm = rowmask + (int64_t)tr * p.W;
     const uint32_t* cm = colmask + (int64_t)tc * p.W;
     int32_t* keys = wkeys[wid];
-    const bool polys = kPoly && F == 1 && floor_free && count >= kPolyMin && (rects || poly_field(p, hdr));
+    const bool polys = kPoly && F == 1 && floor_free && count >= kPolyMin && poly_field(p, hdr, rects != nullptr);
     int64_t done = 0;
     for (int32_t w0 = 0; w0 < p.W; w0 += 64) {
       const int32_t w = w0 + lane;
@@ -2468,7 +2484,7 @@ __device__ __forceinline__ void render16x2_body(
     // FMAs a coefficient and the 64 lanes' reduction; tiles of fewer than kPolyMin Gaussians pass by.
     // The tiles' wide Gaussians as a polynomial each, 64 of the tile's at a time through a queue of (id, place in the
     // row list); they are marked by their place and left out of that tile below.
-    if (floor_free && max(cnt_a, cnt_b) >= kPolyMin) {  // wave-uniform
+    if (floor_free && max(cnt_a, cnt_b) >= kPolyMin && poly_field(p, hdr, true)) {  // wave-uniform
       int32_t* queue = reinterpret_cast<int32_t*>(r16_rows_wevals[wid]);
       wide_bits[lane] = 0u;
       wave_sync();
@@ -2851,7 +2867,7 @@ __device__ inline RowBin bin_tile_row(const Problem& p, const int4* __restrict__
 // row list at their rank (the mask words' popcounts before its word, then its lane's rank in
 // the word), with their column ranges; after a second barrier each wave renders its pair from
 // the list (render16x2_body<kRows>), which also gives the segment starts in closed form.
-// kPoly: the tiles' wide Gaussians as polynomials, where the id capacity has room for a field of them (poly_pairs;
+// kPoly: the tiles' wide Gaussians as polynomials, where the id capacity has room for a field of them (poly_room;
 // without the search 57 registers, not 63, and trained 1280x1280 K = 1024 8.9 us instead of 9.0).
 template <bool kPoly>
 __global__ __launch_bounds__(kRowsThreads) void k_render16x2_rows(
@@ -5262,8 +5278,9 @@ static int forward_render(const gf_field_config* cfg, int64_t out_features, int6
   if (quad_render(p)) {
     if (rows_in_render(p)) {
       const int32_t cp = (p.C + 1) / 2, G = (cp + kRowsThreads / 64 - 1) / (kRowsThreads / 64);
-      hipLaunchKernelGGL((poly_pairs(p, ids_capacity) ? k_render16x2_rows<true> : k_render16x2_rows<false>), dim3((unsigned)((int64_t)p.R * G)), dim3(kRowsThreads), 0, st, p,
-                         row_coords, col_coords, ev, tile_ptr, gaussian_ids_sorted, ids_capacity, delta, ws,
+      auto rows = poly_room(p, ids_capacity) ? k_render16x2_rows<true> : k_render16x2_rows<false>;
+      hipLaunchKernelGGL(rows, dim3((unsigned)((int64_t)p.R * G)), dim3(kRowsThreads), 0, st, p, row_coords,
+                          col_coords, ev, tile_ptr, gaussian_ids_sorted, ids_capacity, delta, ws,
                          reinterpret_cast<const int4*>(ws + L.rect));
       GF_LAUNCH_CHECK("k_render16x2_rows");
       return GF_OK;
@@ -5292,7 +5309,7 @@ static int forward_render(const gf_field_config* cfg, int64_t out_features, int6
     }
     auto render = k_render16<false, false>;
     if (xh > 0) render = k_render16<true, false>;
-    else if (binned_here && poly_pairs(p, ids_capacity)) render = k_render16<false, true>;
+    else if (binned_here && poly_room(p, ids_capacity)) render = k_render16<false, true>;
     hipLaunchKernelGGL(render, dim3((unsigned)(xh + quad_grid(p))),
                        dim3(kTileThreads), 0, st, p, row_coords, col_coords, ev, tile_ptr, gaussian_ids_sorted,
                        ids_capacity, delta, ws, reinterpret_cast<const uint32_t*>(ws + L.rowmask),
@@ -5696,7 +5713,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
   BatchHeader h{};
   std::vector<BatchLayer> ls(n);
   int64_t tile_blocks = 0, emit_blocks = 0, finish_blocks = 0, render_blocks = 0, wide_blocks = 0;
-  bool backward_buffers = true, grads_set = true, tile_render = false, wide_pairs = false;
+  bool backward_buffers = true, grads_set = true, tile_render = false, poly_launch = false, wide_pairs = false;
   for (size_t i = 0; i < n; ++i) {
     const gf_layer& in = layers[i];
     BatchLayer& ly = ls[i];
@@ -5779,10 +5796,12 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
     ly.mo.merged = in.merged_weight;
     ly.mo.scale = in.merged_weight ? in.delta_scale : 1.0f;
     ly.grad_scale = ly.mo.scale;
-    if (ly.pair_render)
+    if (ly.pair_render) {
       render_blocks += ((int64_t)ly.p.R * ((ly.p.C + 1) / 2) + kTileThreads / 64 - 1) / (kTileThreads / 64);
-    else
+    } else {
       tile_render = true;
+      poly_launch = poly_launch || poly_room(ly.p, in.ids_capacity);
+    }
     const int64_t per_emit_block = (kEmitThreads / 64) * (64 / kEmitLanesBatch);
     if (ly.p.W == 0 || pc.W == 0) emit_blocks += (kc + per_emit_block - 1) / per_emit_block;  // emission path
     finish_blocks += (kc * ly.p.S + kTileThreads - 1) / kTileThreads;
@@ -5799,7 +5818,7 @@ int gf_batch_plan(const gf_field_config* cfg, const gf_layer* layers, int32_t n_
   info->emit_blocks = emit_blocks;
   info->finish_blocks = finish_blocks;
   info->render_blocks = render_blocks;
-  info->tile_render = tile_render ? 1 : 0;
+  info->tile_render = tile_render ? (poly_launch ? 2 : 1) : 0;
   info->wide_blocks = wide_pairs ? (int32_t)wide_blocks : 0;
   info->plan_bytes = need;
   if (!plan) return GF_OK;  // size query
@@ -5851,7 +5870,7 @@ int gf_batch_forward(const void* plan, const gf_batch_info* info, uint32_t phase
       GF_LAUNCH_CHECK("k_render16x2_batch");
     }
     if (info->tile_render) {
-      hipLaunchKernelGGL((info->wide_blocks > 0 ? k_render16_batch<true> : k_render16_batch<false>),
+      hipLaunchKernelGGL((info->tile_render == 2 ? k_render16_batch<true> : k_render16_batch<false>),
                          dim3((unsigned)info->tile_blocks), dim3(kTileThreads), 0, st, pl);
       GF_LAUNCH_CHECK("k_render16_batch");
     }

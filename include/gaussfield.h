@@ -387,7 +387,10 @@ typedef struct gf_batch_info {
                                     quadratic-form moments (at 80 and above they are below e^-40) */
   int64_t render_blocks;         /* workgroups of the tile-pair render: 4 pairs of 16x16 tiles each */
   int32_t tile_render;           /* 1: some layer renders tile by tile (32x32 tiles, or a k capacity
-                                    past the masks), a second launch over the tile map */
+                                    past the masks), a second launch over the tile map;
+                                    2: and some layer's id capacity has room for a field of wide
+                                    Gaussians at its k, which that launch then looks for (a launch
+                                    captured in a graph stays as it was captured) */
   int32_t wide_blocks;           /* workgroups of the wide-Gaussian reduction (0: no layer's id capacity
                                     has room for a wide field's pairs) */
 } gf_batch_info;

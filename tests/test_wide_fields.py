@@ -203,6 +203,50 @@ def test_wide_gaussians_on_blocks_of_one_row(M, Nf, K, backward, device):
             grad_close(a, b, name, rtol=1e-5)
 
 
+def _few_wide(M: int, Nf: int, K: int, wide: int, seed: int, around: float | None = None) -> wl.FieldProblem:
+    """`wide` Gaussians of 0.7 of the square (0.3 around one place), the others a few elements wide."""
+    p = init_problem(M, Nf, K, seed, sigma=0.7 if around is None else 0.3)
+    if around is not None:
+        p.mu = (around * torch.randn(K, 2, generator=torch.Generator().manual_seed(seed))).contiguous()
+    sub = p.chol_raw[wide:]
+    p.chol_raw[wide:] = torch.stack((torch.full_like(sub[:, 0], math.log(math.expm1(8.0 / M))), torch.zeros_like(sub[:, 1]),
+                                     torch.full_like(sub[:, 2], math.log(math.expm1(8.0 / Nf)))), dim=-1)
+    return p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Nf,K,wide,tile,around", [
+    (320, 320, 256, 26, 32, None),  # lists of wide Gaussians, small means: element by element
+    (320, 320, 256, 26, 16, None), (320, 320, 1000, 30, 16, None),
+    (320, 320, 256, 60, 32, None),
+    (1280, 1280, 40, 40, 32, 0.02), (1280, 1280, 256, 256, 32, None), (1280, 1280, 300, 300, 16, None)])  # polynomials
+def test_render_bits_do_not_depend_on_the_id_capacity(M, Nf, K, wide, tile, around, device):
+    """The id capacity is the size of a buffer: the same field has the same delta-W, bit for bit, with exactly the room
+    it needs, with more, and with a Gaussian on every tile; in a plan, a plan of a live K and a batch."""
+    from guass_amd.ops import FieldBatchPlan, FieldPlan, StaticFieldPlan
+
+    p = _few_wide(M, Nf, K, wide, 5, around)
+    q = p.to(device)
+    args, kw = (q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp), dict(tile_out=tile, tile_in=tile)
+    default = FieldPlan(M, Nf, K, device, **kw)
+    want = default.forward(*args).clone()
+    pairs = default.pairs()
+    assert default.status() == 0
+    for cap in (pairs, 2 * pairs, 40 * pairs):
+        plan = FieldPlan(M, Nf, K, device, ids_capacity=cap, **kw)
+        assert torch.equal(plan.forward(*args), want), cap
+        assert torch.equal(plan.tile_ptr, default.tile_ptr) and torch.equal(plan.ids[:pairs], default.ids[:pairs])
+    static = StaticFieldPlan(M, Nf, K + 3 if K + 3 <= 256 or K > 256 else K, device, ids_capacity=pairs, **kw)
+    static.set_params(q.mu, q.chol_raw, q.amp)
+    assert torch.equal(static.forward(q.row_coords, q.col_coords), want)
+    out = []
+    for cap in (pairs, 40 * pairs):
+        batch = FieldBatchPlan([q], device, capacities=[cap], **kw)
+        batch.forward()
+        out.append(batch.plans[0].delta.clone())
+    assert torch.equal(out[0], out[1])
+
+
 def _exponents(p: wl.FieldProblem, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """Each Gaussian's exponent q [K, len(x), len(y)] in float64."""
     raw, mu = p.chol_raw.double().to(x.device), p.mu.double().to(x.device)
