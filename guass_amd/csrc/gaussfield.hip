@@ -2098,16 +2098,27 @@ __device__ __forceinline__ void render16_body(
       return u;
     };
     if (__builtin_amdgcn_ballot_w64(lane < nj && my.gen != 0.0f) == 0) {
-      // Four at a time, their LDS reads together, where the chunk is long (1280x5120 K = 4096 clustered, 32x32 tiles:
-      // 33 -> 30 us; chunks of two or three lose 1 us of 16 to it, and the polynomials need its registers).
-      if (!kPoly && floor_free && nj >= 8)
-#pragma clang loop unroll_count(4)
-        for (int j = 0; j < nj; ++j) accumulate_free(at(j));
-      else if (floor_free)
+      // Four at a time, their LDS reads together, where the chunk is long, out of the way of the short ones' code
+      // (1280x5120 on 32x32 tiles: K = 4096 clustered 30.5 -> 24.6 us, K = 2048 trained 16.2 and 16.6; between the
+      // short ones' instructions it took the second to 17.4.  The polynomials need its registers).
+      if (!kPoly && floor_free && __builtin_expect(nj >= 8, 0)) {
+        int j = 0;
+#pragma clang loop unroll(disable)
+        for (; j + 4 <= nj; j += 4) {
+          const GaussEval u0 = at(j), u1 = at(j + 1), u2 = at(j + 2), u3 = at(j + 3);
+          accumulate_free(u0);
+          accumulate_free(u1);
+          accumulate_free(u2);
+          accumulate_free(u3);
+        }
+#pragma clang loop unroll(disable)
+        for (; j < nj; ++j) accumulate_free(at(j));
+      } else if (floor_free) {
 #pragma clang loop unroll(disable)
         for (int j = 0; j < nj; ++j) accumulate_free(at(j));
-      else
+      } else {
         for (int j = 0; j < nj; ++j) accumulate(at(j), std::false_type{});
+      }
     } else {
       for (int j = 0; j < nj; ++j) accumulate(at(j), std::true_type{});
     }
@@ -2923,7 +2934,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
 }
 
 template <bool kHeavy, bool kPoly>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_render16(
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(kPoly ? 7 : 1))) void k_render16(
     Problem p, const float* __restrict__ row_coords, const float* __restrict__ col_coords,
     const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr, int64_t* ids,
     int64_t capacity, float* __restrict__ delta, uint8_t* ws, const uint32_t* __restrict__ rowmask,
@@ -4709,7 +4720,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_batch(const uint8_t* __re
 // Layers rendered tile by tile (BatchLayer::pair_render == 0: 32x32 tiles, or 16x16 tiles whose
 // capacity reaches the emission path), over the tile map; the other layers' blocks return.
 template <bool kPoly>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_render16_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(kPoly ? 7 : 1))) void k_render16_batch(const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   const uint32_t blk = blockIdx.x;
