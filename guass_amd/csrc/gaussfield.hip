@@ -143,8 +143,11 @@ __device__ inline int64_t live_k(const Problem& p) {
 }
 
 // The pair count the backward's saved-state checks use: num_pairs, or in capacity mode the
-// forward's device value.
-__device__ inline int64_t live_pairs(const Problem& p, int64_t num_pairs) { return p.pdev ? *p.pdev : num_pairs; }
+// forward's device value, up to num_pairs (the id capacity: P counts the pairs past it too, which
+// were never emitted and have no room in the id buffer).
+__device__ inline int64_t live_pairs(const Problem& p, int64_t num_pairs) {
+  return p.pdev ? min(*p.pdev, num_pairs) : num_pairs;
+}
 
 // A Gaussian's mean coordinate i (0: row, 1: column) as the field uses it.
 __device__ inline float mu_at(const Problem& p, const float* __restrict__ mu, int64_t i) {
@@ -5367,8 +5370,8 @@ int gf_backward_reduce(const gf_field_config* cfg, int64_t out_features, int64_t
                          workspace, workspace_bytes, stream, nullptr, nullptr);
 }
 
-// kdev / pdev: capacity mode (k is the capacity; see Problem::kdev); num_pairs then only bounds
-// the launch (its heavy-tile and dense-tile choices).
+// kdev / pdev: capacity mode (k is the capacity; see Problem::kdev); num_pairs is then the id
+// capacity, which bounds the launch (its heavy-tile and dense-tile choices) and the pairs read.
 static int backward_reduce(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,
                            const float* grad_delta, const float* row_coords, const float* col_coords,
                            const float* mu, const float* chol_raw, const void* tile_ptr, int32_t tile_ptr_is_int64,

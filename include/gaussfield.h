@@ -271,7 +271,8 @@ int gf_backward_direct(const gf_field_config* cfg, int64_t out_features, int64_t
  * the new K before replaying.  Outputs as gf_forward / gf_backward_direct for the live field (the
  * gradient slots of Gaussians 0 .. *k_dev - 1).  The mask path only: 16x16 or 32x32 tiles,
  * 1 <= k_capacity <= 8192; other fields are refused with GF_E_INVALID_ARGUMENT.  ids_capacity bounds
- * the pairs of every live K (pairs past it are dropped and GF_STATUS_CAPACITY is set).
+ * the pairs of every live K (pairs past it are dropped and GF_STATUS_CAPACITY is set; the backward
+ * leaves them out too and sets its tile_ptr bits).
  */
 int gf_forward_kcap(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k_capacity,
                     const int64_t* k_dev, const float* row_coords, const float* col_coords, const float* mu,

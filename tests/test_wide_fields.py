@@ -435,3 +435,35 @@ def test_wide_field_backward_checks_saved_state(device):
         with pytest.raises(RuntimeError, match=msg):
             ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, t, i, *args,
                                         forward_workspace=ws)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Nf,K,tile,kind", [
+    (320, 330, 300, 16, "narrow"), (320, 330, 300, 32, "narrow"),  # one launch, and the reduction element by element
+    (800, 810, 70, 16, "init"), (800, 810, 70, 32, "init")])  # by moments
+def test_live_k_backward_past_the_id_capacity(M, Nf, K, tile, kind, device):
+    """A plan of a live K whose pairs do not fit: the backward reads the ids that have room, as a plan of the same
+    capacity does, and says so in its status."""
+    from guass_amd.ops import FieldPlan, StaticFieldPlan
+
+    p = init_problem(M, Nf, K, 15) if kind == "init" else _few_wide(M, Nf, K, 0, 15)
+    q = p.to(device)
+    kw = dict(tile_out=tile, tile_in=tile)
+    args = (q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp)
+    whole = FieldPlan(M, Nf, K, device, **kw)
+    whole.forward(*args)
+    cap = whole.pairs() - 32
+    if kind == "init":
+        assert cap * (4 if tile == 32 else 1) >= 480 * K and cap >= 24 * whole.T  # the wide backward's rule
+    plan = FieldPlan(M, Nf, K, device, ids_capacity=cap, **kw)
+    plan.forward(*args)
+    want = [v.clone() for v in plan.backward_direct(q.grad, *args)]
+    static = StaticFieldPlan(M, Nf, K, device, ids_capacity=cap, **kw)
+    static.set_params(q.mu, q.chol_raw, q.amp)
+    static.forward(q.row_coords, q.col_coords)
+    got = static.backward_direct(q.grad, q.row_coords, q.col_coords)
+    assert static.status() == plan.status() and static.status() & N.GF_STATUS_CAPACITY
+    assert static.status("backward") == plan.status("backward") != 0
+    assert static.pairs() == cap + 32
+    for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), got, want):
+        grad_close(a, b.double().cpu(), name, rtol=1e-5)
