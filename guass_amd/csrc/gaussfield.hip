@@ -4937,8 +4937,12 @@ template <typename TP, typename GI>
 void launch_bwd(const Problem& p, dim3 grid, hipStream_t st, const float* grad, const float* rc,
                 const float* cc, const float* mu, const float* raw, const GaussEval* ev,
                 const void* tile_ptr, const void* gids, int64_t num_pairs, uint8_t* ws,
-                const BwdLayout& L, const int32_t* heavy_list, const uint32_t* heavy_count,
+                const BwdLayout& L, const int32_t* heavy_list, const uint32_t* heavy_count, bool counted,
                 const float4* dcoef = nullptr, float* dgrad = nullptr) {
+  // counted: num_pairs is the field's own count.  Where it may be a bound (an id capacity, which says nothing of the
+  // field), the tiles take it: the device deciding instead leaves launches that find nothing to do and a test in
+  // every workgroup of the others (1280x5120 K = 2048 trained, room for every pair: step 59 us by tiles, 68-73 so,
+  // 137 by moments and the rest; 1280x1280 K = 1024 28, 31-32, 56).
   // (the one-launch gradients, dgrad, take the row sums: up to 16 pairs a tile)
   const bool dense = !dgrad && bwd_dense(p, num_pairs);
   // heavy-tile workgroups only with the forward's tile list (the forward workspace)
@@ -4946,7 +4950,7 @@ void launch_bwd(const Problem& p, dim3 grid, hipStream_t st, const float* grad, 
   const TP* tp = reinterpret_cast<const TP*>(tile_ptr);
   const GI* gi = reinterpret_cast<const GI*>(gids);
   if constexpr (std::is_same<TP, int64_t>::value && std::is_same<GI, int64_t>::value) {
-    if (ev && dense && wide_field(p, num_pairs)) {
+    if (counted && ev && dense && wide_field(p, num_pairs)) {
       Problem q = p;
       q.heavy = 0;
       auto wide = p.tile_out == 32 ? k_bwd_wide<true> : k_bwd_wide<false>;
@@ -5357,7 +5361,7 @@ static int backward_reduce(const gf_field_config* cfg, int64_t out_features, int
                            const float* mu, const float* chol_raw, const void* tile_ptr, int32_t tile_ptr_is_int64,
                            const void* gaussian_ids, int32_t ids_is_int64, int64_t num_pairs,
                            const void* forward_workspace, void* workspace, size_t workspace_bytes, void* stream,
-                           const int64_t* kdev, const int64_t* pdev);
+                           const int64_t* kdev, const int64_t* pdev, bool counted);
 
 int gf_backward_reduce(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,
                        const float* grad_delta, const float* row_coords, const float* col_coords,
@@ -5367,17 +5371,18 @@ int gf_backward_reduce(const gf_field_config* cfg, int64_t out_features, int64_t
                        size_t workspace_bytes, void* stream) {
   return backward_reduce(cfg, out_features, in_features, k, grad_delta, row_coords, col_coords, mu, chol_raw,
                          tile_ptr, tile_ptr_is_int64, gaussian_ids, ids_is_int64, num_pairs, forward_workspace,
-                         workspace, workspace_bytes, stream, nullptr, nullptr);
+                         workspace, workspace_bytes, stream, nullptr, nullptr, false);
 }
 
 // kdev / pdev: capacity mode (k is the capacity; see Problem::kdev); num_pairs is then the id
 // capacity, which bounds the launch (its heavy-tile and dense-tile choices) and the pairs read.
+// counted: as for launch_bwd.
 static int backward_reduce(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,
                            const float* grad_delta, const float* row_coords, const float* col_coords,
                            const float* mu, const float* chol_raw, const void* tile_ptr, int32_t tile_ptr_is_int64,
                            const void* gaussian_ids, int32_t ids_is_int64, int64_t num_pairs,
                            const void* forward_workspace, void* workspace, size_t workspace_bytes, void* stream,
-                           const int64_t* kdev, const int64_t* pdev) {
+                           const int64_t* kdev, const int64_t* pdev, bool counted) {
   Problem p;
   int rc = make_problem(cfg, out_features, in_features, k, &p);
   if (rc) return rc;
@@ -5401,13 +5406,13 @@ static int backward_reduce(const gf_field_config* cfg, int64_t out_features, int
   const uint32_t* heavy_count = fws ? &reinterpret_cast<const WsHeader*>(fws)->heavy : nullptr;
   const dim3 grid((unsigned)T);
   if (tile_ptr_is_int64 && ids_is_int64)
-    launch_bwd<int64_t, int64_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count);
+    launch_bwd<int64_t, int64_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
   else if (tile_ptr_is_int64)
-    launch_bwd<int64_t, int32_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count);
+    launch_bwd<int64_t, int32_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
   else if (ids_is_int64)
-    launch_bwd<int32_t, int64_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count);
+    launch_bwd<int32_t, int64_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
   else
-    launch_bwd<int32_t, int32_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count);
+    launch_bwd<int32_t, int32_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
   GF_LAUNCH_CHECK("k_bwd");
   return GF_OK;
 }
@@ -5459,9 +5464,9 @@ int gf_backward(const gf_field_config* cfg, int64_t out_features, int64_t in_fea
                 int64_t num_pairs, float* d_mu, float* d_chol_raw, float* d_amp,
                 const void* forward_workspace, void* workspace, size_t workspace_bytes, void* stream) {
   if (k > 0 && !amp) return set_err(GF_E_INVALID_ARGUMENT, "amp must not be NULL");
-  int rc = gf_backward_reduce(cfg, out_features, in_features, k, grad_delta, row_coords, col_coords,
-                              mu, chol_raw, tile_ptr, tile_ptr_is_int64, gaussian_ids, ids_is_int64,
-                              num_pairs, forward_workspace, workspace, workspace_bytes, stream);
+  int rc = backward_reduce(cfg, out_features, in_features, k, grad_delta, row_coords, col_coords, mu, chol_raw,
+                           tile_ptr, tile_ptr_is_int64, gaussian_ids, ids_is_int64, num_pairs, forward_workspace,
+                           workspace, workspace_bytes, stream, nullptr, nullptr, true);
   if (rc) return rc;
   return gf_backward_finish(cfg, out_features, in_features, k, chol_raw, amp, d_mu, d_chol_raw, d_amp,
                             forward_workspace, workspace, workspace_bytes, stream);
@@ -5542,7 +5547,7 @@ static int backward_direct(const gf_field_config* cfg, int64_t out_features, int
   if (!direct) {
     rc = backward_reduce(cfg, out_features, in_features, k, grad_delta, row_coords, col_coords, mu, chol_raw,
                          tile_ptr, 1, gaussian_ids, 1, num_pairs, forward_workspace, workspace, workspace_bytes,
-                         stream, kdev, pdev);
+                         stream, kdev, pdev, max_span >= 0);
     if (rc) return rc;
     return backward_finish(cfg, out_features, in_features, k, chol_raw, amp, dg + 1, dg + 3, dg, forward_workspace,
                            workspace, workspace_bytes, stream, 8, kdev);
@@ -5563,7 +5568,7 @@ static int backward_direct(const gf_field_config* cfg, int64_t out_features, int
                                mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs,
                                reinterpret_cast<uint8_t*>(workspace), L,
                                reinterpret_cast<const int32_t*>(fws + FL.fill),
-                               &reinterpret_cast<const WsHeader*>(fws)->heavy,
+                               &reinterpret_cast<const WsHeader*>(fws)->heavy, false,
                                reinterpret_cast<const float4*>(fws + FL.dcoef), dg);
   GF_LAUNCH_CHECK("k_bwd");
   return GF_OK;

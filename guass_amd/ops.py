@@ -139,7 +139,8 @@ class FieldPlan:
 
     def backward_reduce(self, grad, row_coords, col_coords, mu, chol_raw, num_pairs: int | None = None,
                         reuse_forward: bool = True):
-        """Per-tile moments.  With ``reuse_forward`` the Gaussian constants come from the last
+        """Per-tile moments, tile by tile whatever ``num_pairs`` (default: the id capacity, a bound).
+        With ``reuse_forward`` the Gaussian constants come from the last
         forward's workspace (same mu / chol_raw), else they are recomputed from mu / chol_raw."""
         n = self.capacity if num_pairs is None else int(num_pairs)
         fwd = self.fwd_ws.data_ptr() if reuse_forward else None
@@ -162,9 +163,28 @@ class FieldPlan:
 
     def backward(self, grad, row_coords, col_coords, mu, chol_raw, amp, num_pairs: int | None = None,
                  reuse_forward: bool = True):
-        """Gradients into ``d_mu``, ``d_chol_raw``, ``d_amp`` from the last forward's binning."""
+        """Gradients into ``d_mu``, ``d_chol_raw``, ``d_amp`` from the last forward's binning.  With its
+        pair count (``num_pairs``, from :meth:`pairs` or :meth:`bin_info`) fields of many wide Gaussians
+        are reduced by their blocks' moments (gf_backward); without, every field tile by tile."""
+        if num_pairs is not None:
+            fwd = self.fwd_ws.data_ptr() if reuse_forward else None
+            N.check(N.lib().gf_backward(ctypes.byref(self.cfg), self.M, self.N, self.K, grad.data_ptr(),
+                                        row_coords.data_ptr(), col_coords.data_ptr(), N.ptr(mu), N.ptr(chol_raw),
+                                        N.ptr(amp), self.tile_ptr.data_ptr(), 1, self.ids.data_ptr(), 1,
+                                        int(num_pairs), N.ptr(self.d_mu), N.ptr(self.d_chol_raw), N.ptr(self.d_amp),
+                                        fwd, self.bwd_ws.data_ptr(), self.bwd_ws_bytes, self._stream()),
+                    "gf_backward")
+            return self.d_mu, self.d_chol_raw, self.d_amp
         self.backward_reduce(grad, row_coords, col_coords, mu, chol_raw, num_pairs, reuse_forward)
         return self.backward_finish(chol_raw, amp, reuse_forward)
+
+    def _pairs_and_span(self, num_pairs: int | None, max_span: int | None) -> tuple[int, int]:
+        """The library's num_pairs and max_span: with both, the field's own; a capacity of 16 pairs a tile or more,
+        which is a bound and rules the one-launch kernel out whatever the span, goes without one."""
+        n = self.capacity if num_pairs is None else int(num_pairs)
+        if max_span is None or (num_pairs is None and n >= 16 * self.T):
+            return n, -1
+        return n, int(max_span)
 
     def backward_direct(self, grad, row_coords, col_coords, mu, chol_raw, amp, num_pairs: int | None = None,
                         max_span: int | None = None):
@@ -175,9 +195,10 @@ class FieldPlan:
         must outlive it.  The gradients are added into the slots (a second call after the same
         forward doubles them).  Fields where the one-launch kernel does not apply run the
         reduction and the finish, which adds into the same slots; so do fields whose widest
-        rectangle ``max_span`` (from :meth:`bin_info`; None: not known) covers 320 tiles or more."""
-        n = self.capacity if num_pairs is None else int(num_pairs)
-        span = -1 if max_span is None else int(max_span)
+        rectangle ``max_span`` (from :meth:`bin_info`; None: not known) covers 320 tiles or more.
+        ``num_pairs`` with ``max_span`` is taken as the field's own pair count (:meth:`bin_info` gives
+        both); without ``max_span`` it may be a bound, and the reduction goes tile by tile."""
+        n, span = self._pairs_and_span(num_pairs, max_span)
         L = N.lib()
         N.check(L.gf_backward_direct(ctypes.byref(self.cfg), self.M, self.N, self.K, grad.data_ptr(),
                                      row_coords.data_ptr(), col_coords.data_ptr(), N.ptr(mu), N.ptr(chol_raw),
@@ -221,8 +242,7 @@ class FieldPlan:
     def direct_launches(self, num_pairs: int | None = None, max_span: int | None = None) -> int:
         """Launches :meth:`backward_direct` makes for ``num_pairs`` (default: the id capacity) and
         ``max_span`` (None: not known): 1, or 2 where it runs the reduction and the finish."""
-        n = self.capacity if num_pairs is None else int(num_pairs)
-        span = -1 if max_span is None else int(max_span)
+        n, span = self._pairs_and_span(num_pairs, max_span)
         r = int(N.lib().gf_backward_direct_launches(ctypes.byref(self.cfg), self.M, self.N, self.K, n, span))
         if r < 0:
             N.check(-r, "gf_backward_direct_launches")

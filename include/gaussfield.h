@@ -193,7 +193,10 @@ int gf_backward(const gf_field_config* cfg, int64_t out_features, int64_t in_fea
                 float* d_mu, float* d_chol_raw, float* d_amp, const void* forward_workspace,
                 void* workspace, size_t workspace_bytes, void* stream);
 
-/* First half of gf_backward (reference backward.cu:592-702: per-pair partials + reduce-by-key). */
+/* First half of gf_backward (reference backward.cu:592-702: per-pair partials + reduce-by-key).
+ * num_pairs may be a bound here, such as the id capacity (tile_ptr then ends below it and the
+ * workspace's status says so): the field is reduced tile by tile, whatever the bound.  gf_backward,
+ * whose num_pairs is the field's own, takes fields of many wide Gaussians by the blocks' moments. */
 int gf_backward_reduce(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,
                        const float* grad_delta, const float* row_coords, const float* col_coords,
                        const float* mu, const float* chol_raw,
@@ -248,7 +251,9 @@ int gf_backward_train(const gf_field_config* cfg, int64_t out_features, int64_t 
  * on its one slot would cost the kernel more than the second launch (about 10 ns a tile), and
  * grids of 8192 tiles or more whose widest rectangle is not known (max_span < 0: graphs
  * captured before the content is; their reduction spreads each Gaussian's atomics over
- * stripes).  The gradients agree with gf_backward's
+ * stripes).  A known max_span also tells that num_pairs, which gf_bin_info gives beside it, is the
+ * field's own: fields of many wide Gaussians then go by the blocks' moments, as in gf_backward; with
+ * max_span < 0 num_pairs may be a bound and they go tile by tile.  The gradients agree with gf_backward's
  * within fp32 rounding (the map is applied per tile, in fp32).
  */
 int gf_backward_direct(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,

@@ -467,3 +467,79 @@ def test_live_k_backward_past_the_id_capacity(M, Nf, K, tile, kind, device):
     assert static.pairs() == cap + 32
     for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), got, want):
         grad_close(a, b.double().cpu(), name, rtol=1e-5)
+
+
+def _flag(plan) -> int:
+    """What a reduction by moments left in the backward workspace's header: whether some Gaussians were not wide."""
+    return int(plan.bwd_ws[4:8].view(torch.int32)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,Nf,K,tile,kind", [
+    (800, 810, 150, 16, "sparse"), (800, 810, 150, 32, "sparse"),  # a few elements wide everywhere
+    (800, 810, 2100, 16, "clustered"),  # heavy tiles, their four-wave workgroups
+    (800, 810, 150, 16, "mixed"), (800, 810, 150, 32, "mixed")])  # wide with some that are not
+def test_bounded_pair_count_goes_by_tiles(M, Nf, K, tile, kind, device):
+    """A pair count that may be a bound (the id capacity, by default a Gaussian on every tile) says nothing of the
+    field: the backward reduces it tile by tile, without a pass by moments before, and also in a replayed graph."""
+    from guass_amd.ops import FieldPlan, StaticFieldPlan
+    from oracle import field_oracle as fo
+
+    if kind == "mixed":
+        p = _mixed(M, Nf, K, 21)
+    else:
+        p = _few_wide(M, Nf, K, 0, 21)
+        if kind == "clustered":
+            at = torch.randn(8, 2, generator=torch.Generator().manual_seed(22)).mul(0.4).clamp(-0.9, 0.9)
+            p.mu = (at[torch.arange(K) % 8] + 0.05 * p.mu).contiguous()
+    r = fo.gaussian_field_fwd_bwd_fp64(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, tile, tile, 3.0,
+                                       False, 80.0)
+    T, P, quad = r[1].numel() - 1, int(r[1][-1]), 4 if tile == 32 else 1
+    by_moments = quad * P >= 480 * K and P >= 24 * T and quad * T >= 2048
+    assert by_moments == (kind == "mixed")
+    q = p.to(device)
+    args, kw = (q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp), dict(tile_out=tile, tile_in=tile)
+    plan = FieldPlan(M, Nf, K, device, **kw)
+    cap = plan.capacity
+    assert quad * cap >= 480 * K and cap >= 24 * T and quad * T >= 2048  # the bound would make any field a wide one
+    plan.forward(*args)
+    pairs, span = plan.bin_info()
+    assert pairs == P
+
+    def close(got):
+        for name, a, b in zip(("d_mu", "d_chol_raw", "d_amp"), got, r[3:]):
+            grad_close(a, b, name, rtol=1e-5)
+
+    plan.backward_reduce(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw)
+    assert _flag(plan) == 0
+    close(plan.backward_finish(q.chol_raw, q.amp))
+    close(plan.backward(q.grad, *args))
+    close(plan.backward(q.grad, *args, num_pairs=P))
+    for num, sp in ((None, None), (None, span), (P, span)):
+        plan.forward(*args)
+        close(plan.backward_direct(q.grad, *args, num_pairs=num, max_span=sp))
+
+    static = StaticFieldPlan(M, Nf, K + 40, device, ids_capacity=cap, **kw)
+    static.set_params(q.mu, q.chol_raw, q.amp)
+
+    def step():
+        plan.forward(*args)
+        a = plan.backward_direct(q.grad, *args, num_pairs=P, max_span=span)
+        static.forward(q.row_coords, q.col_coords)
+        return a, static.backward_direct(q.grad, q.row_coords, q.col_coords)
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        step()
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        a, b = step()
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        close(a)
+        close([v[:K] for v in b])
+        q.amp.add_(0.0)  # the program's own work between the replays
+    assert plan.status() == 0 and static.status() == 0
