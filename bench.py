@@ -728,7 +728,7 @@ def main() -> int:
     }
     if not batched:
         out["config"]["max_span"] = span
-        out["config"]["backward_launches"] = 1 if direct_one else 2
+        out["config"]["backward_launches"] = plan.direct_launches(P, span)
     if not batched and plan.fused_supported(span):
         out["fused"] = fused_times(plan, q, total, per_run, args, graph_time_us, ph["k_bin"])
     if not batched and args.dropin_calls > 0:

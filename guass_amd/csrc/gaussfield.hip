@@ -5497,7 +5497,9 @@ int gf_backward_direct_launches(const gf_field_config* cfg, int64_t out_features
   Problem p;
   int rc = make_problem(cfg, out_features, in_features, k, &p);
   if (rc) return -rc;
-  return direct_one_launch(p, num_pairs, max_span) && k > 0 ? 1 : 2;
+  if (direct_one_launch(p, num_pairs, max_span) && k > 0) return 1;
+  // the reduction (by tiles, or by moments with what they leave) and the finish
+  return max_span >= 0 && wide_field(p, num_pairs) ? 3 : 2;
 }
 
 size_t gf_forward_grads_offset(int64_t out_features, int64_t in_features, int64_t k,

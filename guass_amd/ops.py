@@ -241,7 +241,8 @@ class FieldPlan:
 
     def direct_launches(self, num_pairs: int | None = None, max_span: int | None = None) -> int:
         """Launches :meth:`backward_direct` makes for ``num_pairs`` (default: the id capacity) and
-        ``max_span`` (None: not known): 1, or 2 where it runs the reduction and the finish."""
+        ``max_span`` (None: not known): 1, 2 where it runs the reduction and the finish, or 3 where the
+        reduction goes by the blocks' moments (a field of many wide Gaussians, by its own pair count)."""
         n, span = self._pairs_and_span(num_pairs, max_span)
         r = int(N.lib().gf_backward_direct_launches(ctypes.byref(self.cfg), self.M, self.N, self.K, n, span))
         if r < 0:

@@ -321,8 +321,9 @@ int gf_fwd_bwd_fused_supported(const gf_field_config* cfg, int64_t out_features,
                                int64_t ids_capacity, int64_t max_span);
 
 /* Kernel launches gf_backward_direct makes for this field, pair count and widest rectangle
- * (max_span < 0: not known): 1 (the direct kernel) or 2 (reduction + finish); the negated error
- * code on an invalid configuration. */
+ * (max_span < 0: not known): 1 (the direct kernel), 2 (reduction + finish) or 3 (the reduction by
+ * the blocks' moments, the one of what they leave, finish); the negated error code on an invalid
+ * configuration. */
 int gf_backward_direct_launches(const gf_field_config* cfg, int64_t out_features, int64_t in_features, int64_t k,
                                 int64_t num_pairs, int64_t max_span);
 

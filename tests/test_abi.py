@@ -168,6 +168,24 @@ def test_backward_direct_host_logic():
     assert rc == GF_E_WORKSPACE
 
 
+def test_backward_direct_launches_by_moments():
+    """Fields of many wide Gaussians by their own pair count (the widest rectangle given with it): two launches of the
+    reduction and the finish, on 16x16 and 32x32 tiles; with a bound, a low clamp or past the masks by tiles."""
+    lib = N.lib()
+
+    def launches(P, span, K=1024, tile=16, clamp=80.0):
+        cfg = N.make_config(tile, tile, 3.0, False, clamp)
+        return lib.gf_backward_direct_launches(ctypes.byref(cfg), 1280, 5120, K, P, span)
+
+    assert launches(480 * 1280, 3000, K=1280) == 3
+    assert launches(480 * 1280 - 1, 3000, K=1280) == 2  # fewer than 480 blocks a Gaussian
+    assert launches(480 * 1280, -1, K=1280) == 2  # the count may be a bound
+    assert launches(24 * 6400, 700, K=1280, tile=32) == 3
+    assert launches(24 * 6400 - 1, 700, K=1280, tile=32) == 2  # fewer than 24 a tile
+    assert launches(480 * 1280, 3000, K=1280, clamp=24.0) == 2
+    assert launches(480 * 9000, 3000, K=9000) == 2
+
+
 def test_bin_info_and_train_backward_host_checks():
     """gf_forward_bin_info / gf_read_bin_info refuse NULL outputs, and gf_backward_train checks
     its field and buffers before any device work on either of its paths (safe without a GPU)."""
