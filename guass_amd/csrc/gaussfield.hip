@@ -3630,7 +3630,50 @@ __host__ __device__ inline bool wide_field(const Problem& p, int64_t pairs, int6
          q * p.R * p.C >= min_blocks && pairs >= kPolyMin * (int64_t)p.R * p.C && q * pairs >= mean_blocks * p.K;
 }
 
-template <bool kQuad>
+// The wide Gaussians that a tile's list names again (a bit each marks them once; every time counts): element by element,
+// a Gaussian a lane, over the 2x2 tiles from (tr0, tc0).  No forward makes such lists.
+__device__ __forceinline__ void wide_again(const Problem& p, const float* __restrict__ grad,
+                                           const float* __restrict__ row_coords, const float* __restrict__ col_coords,
+                                           const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr,
+                                           const int64_t* __restrict__ gids, int64_t P, int32_t tr0, int32_t tc0,
+                                           uint32_t fits, const WideLds& w, uint32_t* bits, int32_t W, float* acc_s) {
+  const int lane = threadIdx.x & 63;
+  for (int32_t i = lane; i < 4 * W; i += 64) bits[i] = 0u;
+  wave_sync();
+  for (int b = 0; b < 4; ++b) {
+    const int32_t tr = tr0 + (b >> 1), tc = tc0 + (b & 1);
+    if (tr >= p.R || tc >= p.C) continue;
+    const int64_t* tp = tile_ptr + ((int64_t)tr * p.C + tc);
+    const PolyBlock pb{w.block[b][0], w.block[b][1], w.block[b][2], w.block[b][3], w.block[b][4], w.block[b][5], 0, 0};
+    for (int64_t j = max(tp[0], (int64_t)0) + lane; j < min(tp[1], P); j += 64) {
+      const int64_t g = gids[j];
+      if (g < 0 || g >= live_k(p)) continue;
+      const uint32_t bit = 1u << (g & 31);
+      if ((atomicOr(bits + (b * W + (g >> 5)), bit) & bit) == 0u) continue;
+      const GaussEval u = load_eval(ev, g);
+      if (!poly_gauss(pb, u).moment || ((fits >> b) & 1u) == 0u) continue;  // k_bwd_rest's
+      float m[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int32_t r = 16 * tr; r < min(16 * tr + 16, p.M); ++r) {
+        const float dx = row_coords[r] - u.mu0, a = u.wa * dx, z0 = u.wb * dx;
+        for (int32_t c = 16 * tc; c < min(16 * tc + 16, p.N); ++c) {
+          const float dy = col_coords[c] - u.mu1, z = fmaf(u.wc, dy, z0);
+          const float h = grad[(int64_t)r * p.N + c] * __builtin_amdgcn_exp2f(-fmaf(z, z, a * a));
+          m[0] += h;
+          m[1] = fmaf(h, dx, m[1]);
+          m[2] = fmaf(h, dy, m[2]);
+          m[3] = fmaf(h * dx, dx, m[3]);
+          m[4] = fmaf(h * dx, dy, m[4]);
+          m[5] = fmaf(h * dy, dy, m[5]);
+        }
+      }
+      for (int k = 0; k < 6; ++k) unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)g + (uint32_t)k), m[k]);
+    }
+  }
+  wave_sync();
+}
+
+// kAgain: the lists are the caller's (a batch's are its own forward's).
+template <bool kQuad, bool kAgain>
 __device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __restrict__ grad,
                                               const float* __restrict__ row_coords,
                                               const float* __restrict__ col_coords,
@@ -3683,6 +3726,7 @@ __device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __r
     set_status(&hdr->status, g < 0 ? GF_STATUS_IDS_NEGATIVE : GF_STATUS_IDS_RANGE);
     return -1;
   };
+  bool again = false;  // (uniform) a list names some Gaussian again
   if constexpr (!kQuad) {  // a bit a listed Gaussian, block by block
     for (int32_t i = lane; i < 4 * W; i += 64) bits[i] = 0u;
     wave_sync();
@@ -3691,9 +3735,12 @@ __device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __r
       const int64_t sb = readlane_i64(s, b), nb = readlane_i64(nl, b);
       for (int64_t j = lane; j < nb; j += 64) {
         const int32_t g = checked_id(sb + j);
-        if (g >= 0) atomicOr(bits + (b * W + (g >> 5)), 1u << (g & 31));
+        if (g < 0) continue;
+        const uint32_t bit = 1u << (g & 31), old = atomicOr(bits + (b * W + (g >> 5)), bit);
+        if (kAgain && (old & bit) != 0u) again = true;
       }
     }
+    if (kAgain) again = __builtin_amdgcn_ballot_w64(again) != 0ull;
   }
   // the blocks' moments
   uint32_t fits = 0u;
@@ -3713,6 +3760,8 @@ __device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __r
     __builtin_amdgcn_sched_barrier(0);
   }
   float* const acc_s = reinterpret_cast<float*>(ws + L.acc) + 8 * acc_slot(p, 0, unit & (p.S - 1));
+  if (kAgain && __builtin_expect(again, 0))
+    wide_again(p, grad, row_coords, col_coords, ev, tile_ptr, gids, P, 2 * ur, 2 * uc, fits, w, bits, W, acc_s);
   bool left = false;
   // nj listed Gaussians, id_of(j) the j-th (negative: none): a lane each, block after block, or from a
   // last 32 or fewer two blocks and from a last 16 or fewer all four at once, a lane a (Gaussian, block).
@@ -3835,7 +3884,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)
   extern __shared__ uint32_t wide_bits[];
   const int64_t unit = (int64_t)blockIdx.x * (kTileThreads / 64) + wave_id();
   if (unit >= wide_units(p)) return;
-  bwd_wide_body<kQuad>(p, grad, row_coords, col_coords, ev, tile_ptr, gids, num_pairs, ws, L, (int32_t)unit,
+  bwd_wide_body<kQuad, !kQuad>(p, grad, row_coords, col_coords, ev, tile_ptr, gids, num_pairs, ws, L, (int32_t)unit,
                        lds[wave_id()], wide_bits + wave_id() * 4 * ((p.K + 31) / 32));
 }
 
@@ -4795,10 +4844,10 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)
   const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
   const GaussEval* ev = reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval);
   if (p.tile_out == 32)
-    bwd_wide_body<true>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
+    bwd_wide_body<true, false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
                         lds[wave_id()], bits[wave_id()]);
   else
-    bwd_wide_body<false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
+    bwd_wide_body<false, false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
                          lds[wave_id()], bits[wave_id()]);
 }
 

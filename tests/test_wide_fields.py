@@ -543,3 +543,29 @@ def test_bounded_pair_count_goes_by_tiles(M, Nf, K, tile, kind, device):
         close([v[:K] for v in b])
         q.amp.add_(0.0)  # the program's own work between the replays
     assert plan.status() == 0 and static.status() == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,tile", [("init", 16), ("mixed", 16), ("init", 32)])
+def test_wide_field_backward_of_ids_listed_again(kind, tile, device):
+    """A saved binning whose lists name a Gaussian more than once: each time counts, by moments as element by element
+    (whose constants are recomputed from the parameters)."""
+    from guass_amd.cuda_field import ext
+
+    M, Nf, K = 800, 810, 150
+    p = _mixed(M, Nf, K, 23) if kind == "mixed" else init_problem(M, Nf, K, 23)
+    q = p.to(device)
+    args = (tile, tile, 3.0, False, 80.0)
+    _, tp, ids, ws = ext.forward_with_workspace(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, *args)
+    T, pairs = tp.numel() - 1, int(tp[-1])
+    assert pairs * (4 if tile == 32 else 1) >= 480 * K and pairs >= 24 * T  # the rule the kernels go by
+    listed = tp.cpu()
+    for t in (0, 1, T // 2, T - 1):
+        s, e = int(listed[t]), int(listed[t + 1])
+        assert e - s >= 8
+        ids[s + 3:e - 1:4] = ids[s + 2].clone()
+        ids[e - 1] = ids[e - 2].clone()
+    a, b = (ext.gaussian_field_backward(q.grad, q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tp, ids, *args,
+                                        forward_workspace=w) for w in (ws, None))
+    for name, x, y in zip(("d_mu", "d_chol_raw", "d_amp"), a, b):
+        grad_close(x, y.double().cpu(), name, rtol=1e-5)
