@@ -84,18 +84,24 @@ def test_striped_reduction_of_few_gaussians(M, Nf, K, tile, device):
             grad_close(a, b, name)
 
 
-def _mixed(M: int, Nf: int, K: int, seed: int) -> wl.FieldProblem:
+def _mixed(M: int, Nf: int, K: int, seed: int, sigma: float | None = None) -> wl.FieldProblem:
     """init_problem with every fifth Gaussian a few elements wide, listed between the others."""
-    p = init_problem(M, Nf, K, seed)
+    p = init_problem(M, Nf, K, seed, sigma)
     sub = p.chol_raw[::5]
     p.chol_raw[::5] = torch.stack((torch.full_like(sub[:, 0], math.log(math.expm1(8.0 / M))), torch.zeros_like(sub[:, 1]),
                                    torch.full_like(sub[:, 2], math.log(math.expm1(8.0 / Nf)))), dim=-1)
     return p
 
 
-# Blocks cut by the matrix's edges, one row and one column of blocks, lists of 24 (the fewest taken), 64, 65 and
-# several times 64, narrow Gaussians between the wide ones, normalised ones, and a clamp that keeps them all
-# element by element.
+def _by_polynomials(tile_ptr, K: int, tile: int) -> bool:
+    """The rule of the renders that look for wide Gaussians, for fields whose widest rectangle is no outlier: 256 blocks
+    a Gaussian or more on average, and a list of 24."""
+    tp = tile_ptr.cpu()
+    return int(tp[-1]) * (4 if tile == 32 else 1) >= 256 * K and int((tp[1:] - tp[:-1]).max()) >= 24
+
+
+# Fields of wide Gaussians, most of them small, whose mean rectangle is below the polynomials' rule ("ragged" and "rows"
+# are above it): element by element, on the lists and grids that the polynomials have to handle too (below).
 WIDE_CASES = {
     "ragged": (250, 333, 200, 32, {}),
     "one_row": (9, 700, 60, 16, {}),
@@ -113,19 +119,47 @@ WIDE_CASES = {
     "rows_one_row": (16, 340, 321, 16, {"normalize": True}),
 }
 
+# Fields that go by polynomials: blocks cut by the matrix's edges, one row and one column of blocks, lists of 24
+# (the fewest taken), 64, 65 and several times 64, narrow Gaussians between the wide ones, normalised ones, and
+# from 257 Gaussians on the pairs of tiles from a row list.
+POLY_CASES = {
+    "ragged": (330, 345, 200, 32, {}),
+    "n24": (320, 320, 24, 32, {}),
+    "n64": (320, 320, 64, 16, {}),
+    "n65": (320, 330, 65, 32, {}),
+    "n65_16": (330, 320, 65, 16, {}),
+    "mixed": (333, 350, 150, 32, {}),
+    "mixed_16": (333, 350, 256, 16, {}),
+    "normalize": (320, 327, 90, 16, {"normalize": True}),
+    "noclamp": (320, 320, 256, 32, {"clamp": None}),
+    "one_row": (16, 4300, 60, 16, {}),
+    "one_column": (4300, 16, 60, 16, {}),
+    "rows": (330, 345, 257, 16, {}),
+    "rows_mixed": (330, 345, 1024, 16, {}),
+    "rows_mixed_few": (320, 333, 290, 16, {"normalize": True}),
+    "rows_one_column": (4300, 16, 300, 16, {}),
+    "rows_one_row": (16, 4300, 321, 16, {"clamp": None}),
+}
+
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", list(WIDE_CASES))
+@pytest.mark.parametrize("case", list(WIDE_CASES) + [f"poly_{c}" for c in POLY_CASES])
 def test_wide_gaussians_render(case, device):
-    """Blocks of wide Gaussians as polynomials against the oracle's exponentials, at the parity bar."""
+    """Fields of wide Gaussians, element by element and as polynomials, against the oracle's exponentials, at the parity
+    bar."""
     from guass_amd.cuda_field import ext
     from oracle import field_oracle as fo
 
-    M, Nf, K, tile, kw = WIDE_CASES[case]
-    p = (_mixed if "mixed" in case else init_problem)(M, Nf, K, 7, **({} if "mixed" in case else {"sigma": max(3.0 / math.sqrt(K), 0.7)}))
+    poly = case.startswith("poly_")
+    M, Nf, K, tile, kw = POLY_CASES[case[5:]] if poly else WIDE_CASES[case]
+    if poly:
+        p = (_mixed if "mixed" in case else init_problem)(M, Nf, K, 7, sigma=1.5)
+    else:
+        p = (_mixed if "mixed" in case else init_problem)(M, Nf, K, 7, **({} if "mixed" in case else {"sigma": max(3.0 / math.sqrt(K), 0.7)}))
     norm, clamp = kw.get("normalize", False), kw.get("clamp", 80.0)
     r = fo.gaussian_field_fwd_bwd_batched(p.row_coords, p.col_coords, p.mu, p.chol_raw, p.amp, p.grad, tile, tile,
                                           3.0, norm, clamp)
+    assert _by_polynomials(r[1], K, tile) == (poly or case in ("ragged", "rows"))
     q = p.to(device)
     delta, tp, ids = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tile, tile, 3.0,
                                                 norm, clamp)
@@ -134,15 +168,18 @@ def test_wide_gaussians_render(case, device):
 
 
 @pytest.mark.gpu
-def test_wide_gaussians_infinite_amplitude(device):
+@pytest.mark.parametrize("M,Nf,K,tile,poly", [(64, 64, 64, 32, False), (320, 320, 64, 32, True), (320, 320, 64, 16, True),
+                                              (320, 320, 300, 16, True)])
+def test_wide_gaussians_infinite_amplitude(M, Nf, K, tile, poly, device):
     """An infinite amplitude among wide Gaussians stays out of the block's polynomial: every element it
     reaches is infinite, not NaN."""
     from guass_amd.cuda_field import ext
 
-    p = init_problem(64, 64, 64, 3, sigma=1.5)
+    p = init_problem(M, Nf, K, 3, sigma=1.5)
     p.amp[10] = float("inf")
     q = p.to(device)
-    delta, _, _ = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, 32, 32, 3.0, False, 80.0)
+    delta, tp, _ = ext.gaussian_field_forward(q.row_coords, q.col_coords, q.mu, q.chol_raw, q.amp, tile, tile, 3.0, False, 80.0)
+    assert _by_polynomials(tp, K, tile) == poly
     assert torch.isposinf(delta).all()
 
 
