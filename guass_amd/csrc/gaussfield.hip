@@ -15,7 +15,8 @@
 //   k_prep also stores the chain-rule maps.  Up to 256 Gaussians each tile's wave bins itself.
 // Emission path, four kernels:
 //   k_prep, k_bin_tiles as above without the constants and the masks, over the tile rows alone;
-//   k_bin      in their place for no Gaussians and for very wide grids, one workgroup per field: rectangles, the pair total, per-tile Gaussian counts
+//   k_bin      in their place for no Gaussians and for very wide grids, one workgroup per field:
+//              rectangles, the pair total, per-tile Gaussian counts
 //              from row-wise difference arrays and their scan -> tile_ptr; every scan runs in
 //              LDS (DPP wave scans) and global memory is only written, coalesced.  (The
 //              batched form, k_bin_batch, one workgroup per field, also builds the masks.)
@@ -31,10 +32,11 @@
 // Wide Gaussians (nearly constant over a 16x16 block) go through the block's polynomial instead of
 // element by element ("Wide Gaussians" below): in k_render16, k_render16x2_rows, k_render16_batch
 // and, for the backward of fields made of them, k_bwd_wide (+ k_bwd_rest for what is not wide).
-// Backward (reference backward.cu:541-716), two kernels:
+// Backward (reference backward.cu:541-716), two kernels (three for a field of wide Gaussians):
 //   k_bwd16    one wave per 16x16 tile: lanes are (Gaussian slot, tile row); each lane sums
 //              16 pixels of its row for its Gaussian into six moments, 16-lane DPP row sums
 //              reduce them, and one atomic per (Gaussian, tile, moment) accumulates them.
+//              (Fields of wide Gaussians, by their own pair count: k_bwd_wide, then k_bwd_rest.)
 //   k_bwd_finish  per Gaussian: chain rule from the six moments to (mu, chol_raw, amp), in
 //              double, then clears the accumulators so the workspace stays zeroed.
 //   (k_bwd_any handles other tile shapes.)
@@ -1173,7 +1175,8 @@ __global__ __launch_bounds__(kTilesThreads) void k_prep(Problem p, const float* 
   }
 }
 
-// kMasks == false (emission path: R workgroups, a tile row each): tile_ptr alone, with the tiles' fill counters cleared.
+// kMasks == false (emission path: R workgroups, a tile row each): tile_ptr alone, with the tiles' fill counters
+// cleared.
 template <bool kMasks, int kThreads>
 __global__ __launch_bounds__(kThreads) void k_bin_tiles(Problem p, int64_t* __restrict__ tile_ptr,
                                                         int64_t* __restrict__ num_pairs, uint8_t* ws, FwdLayout L,
@@ -1660,8 +1663,8 @@ constexpr int kPolyMore = 8;  // and a further 64's, whose sums join the first's
 constexpr float kPolyMaxQ = 24.0f;
 constexpr float kPolyMaxAmp = 1e30f;  // amplitudes past this (infinite ones) go element by element
 
-// The tile renders look for wide Gaussians where the mean rectangle covers kPolyBlocks blocks or more (fresh layers, 8 in
-// a batch on 32x32 tiles, with the search and without: 640x640 at 349 blocks 47 and 59 us, at 259 64 and 62, 320x320 at
+// The tile renders look for wide Gaussians where the mean rectangle covers kPolyBlocks blocks or more (fresh layers, 8
+// in a batch on 32x32 tiles, with the search and without: 640x640 at 349 blocks 47 and 59 us, at 259 64 and 62, 320x320 at
 // 268 21 and 25, at 215 26.2 and 26.5) and, as far as the binning before the render tells, none is kPolySpread times
 // the mean (many small and few huge ones: the search costs more than it finds, 1280x5120 K = 4096 on 32x32 tiles with
 // heavy-tailed log-scales 136 -> 147 us).  The kernels go by the field's own pairs and rectangles (poly_field), so that
@@ -1777,7 +1780,8 @@ __device__ __forceinline__ void poly_coefs(const PolyGauss& o, float c00, Emit&&
 #pragma unroll
   for (int a = 0; a <= D + X; ++a) {
     float cur[D + 1];
-    const float n1 = a > 0 ? o.L1 * (-1.0f / (a > 0 ? a : 1)) : 0.0f, n2 = a > 1 ? o.Q11x2 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
+    const float n1 = a > 0 ? o.L1 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
+    const float n2 = a > 1 ? o.Q11x2 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
     const float n3 = a > 0 ? o.Q12 * (-1.0f / (a > 0 ? a : 1)) : 0.0f;
 #pragma unroll
     for (int b = 0; b <= D + X - a; ++b) {
@@ -1841,7 +1845,8 @@ __device__ __forceinline__ void poly_sum_add(PolySum& ps, PolyGauss o, bool in, 
 
 // The polynomial of the sums at the lane's elements: row lane / 4, columns 4 (lane % 4) .. + 3, whose offsets
 // xi (row) and eta (columns) are given.  lds: 128 floats of the wave's.
-__device__ __forceinline__ void poly_eval(const PolySum& ps, float xi, const float (&eta)[4], float* lds, float (&out)[4]) {
+__device__ __forceinline__ void poly_eval(const PolySum& ps, float xi, const float (&eta)[4], float* lds,
+                                          float (&out)[4]) {
   const int lane = opaque_lane();
   const bool hb0 = (lane & 1) != 0, hb1 = (lane & 2) != 0;
   // each register over its rows' lanes by recursive halving (as the backward's moments): lane bits
@@ -2248,7 +2253,8 @@ __device__ __forceinline__ void render16_body(
             const bool stay = mine && !(add && wide);
             const uint64_t bal = __builtin_amdgcn_ballot_w64(stay);
             if (stay)  // (at or before its place, which every lane has read)
-              keys[left + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = key;
+              keys[left + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = key;
             left += __popcll(bal);
             if (!add) continue;
             if (!marked) {
@@ -2494,7 +2500,7 @@ __device__ __forceinline__ void render16x2_body(
   bool marked = false;
   if constexpr (kRows && kPoly) {
     // The polynomials come before the loop over the row list and leave only their sums in registers (63 in all, as the
-    // occupancy needs): 1280x5120 K = 1024, fresh (70 Gaussians an element), render 98 -> 61 us.  What remains is three
+    // occupancy needs): 1280x5120 K = 1024, fresh (70 Gaussians an element), render 95 -> 60 us.  What remains is three
     // FMAs a coefficient and the 64 lanes' reduction; tiles of fewer than kPolyMin Gaussians pass by.
     // The tiles' wide Gaussians as a polynomial each, 64 of the tile's at a time through a queue of (id, place in the
     // row list); they are marked by their place and left out of that tile below.
@@ -2519,7 +2525,8 @@ __device__ __forceinline__ void render16x2_body(
             const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
             if (in)
               queue[pend + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = e.x | (j << 16);
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] =
+                  e.x | (j << 16);
             pend += __popcll(bal);
             j0 += 64;
           }
@@ -2896,8 +2903,8 @@ __global__ __launch_bounds__(kRowsThreads) void k_render16x2_rows(
   const int32_t pc = ((int32_t)blockIdx.x - tr * G) * kWaves + wave_id();  // the wave's pair
   const RowBin rb = bin_tile_row<kRowsThreads>(p, rects, tr, rl, tile_ptr);
   if (pc >= cp) return;  // past the row's last pair (no barrier follows)
-  render16x2_body<false, true, kPoly>(p, row_coords, col_coords, ev, nullptr, ids, capacity, delta, ws, nullptr, nullptr,
-                               tr, 2 * pc, nullptr, MergedOut{nullptr, nullptr, 1.0f}, 0u, rb);
+  render16x2_body<false, true, kPoly>(p, row_coords, col_coords, ev, nullptr, ids, capacity, delta, ws, nullptr,
+                                      nullptr, tr, 2 * pc, nullptr, MergedOut{nullptr, nullptr, 1.0f}, 0u, rb);
 }
 
 // Single 16x16 fields on the mask path with heavy-tile workgroups: the first workgroups take one
@@ -3287,13 +3294,15 @@ __device__ __forceinline__ void bwd16_body(
         myg = (int32_t)g;
       }
     }
-    const uint64_t skip = kRest && grad_fits ? __builtin_amdgcn_ballot_w64(myg >= 0 && poly_gauss(pb, my).moment) : 0ull;
+    const uint64_t skip =
+        kRest && grad_fits ? __builtin_amdgcn_ballot_w64(myg >= 0 && poly_gauss(pb, my).moment) : 0ull;
     if (kRest && skip != 0ull) {
       // the others to the front, in order
       const bool rest = ((skip >> lane) & 1ull) == 0 && lane < nj;
       const uint64_t rbal = __builtin_amdgcn_ballot_w64(rest);
       nj = __popcll(rbal);
-      const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(rbal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)rbal, 0u));
+      const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(rbal >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)rbal, 0u));
       const int to = (rest ? below : nj + lane - below) << 2;
       auto send = [&](float f) { return __int_as_float(__builtin_amdgcn_ds_permute(to, __float_as_int(f))); };
       my.mu0 = send(my.mu0);
@@ -3600,8 +3609,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
 // Device-wide float atomics run at about 160 lanes' adds a nanosecond on the whole chip here: 11 million of
 // them (six a Gaussian and block) held a 1280x5120 field of 1024 wide Gaussians at 120 us in a form with a block a
 // wave, where the same kernel without its atomics took 50; four blocks' sums make a quarter of the adds.
-// Reductions, element by element -> this and the rest: that field 176 -> 56 us, 1280x1280 K = 256 on 32x32 tiles
-// 37 -> 22 us, 28 layers of K = 256 366 -> 105 us (all of it was 743 -> 267 us with the render's polynomials).
+// Reductions, element by element -> this and the rest: that field 178 -> 64 and 5 us, 1280x1280 K = 256 on 32x32 tiles
+// 35 -> 22 and 4, 28 layers of K = 256 366 -> 137 and 19 (and 28 for their layers of 320, element by element).
 constexpr int kWideKeys = 256;
 struct WideLds {            // a wave's
   float gt[16 * kWideRow];  // a block's dL/d(delta-W); later the moments on their way out
@@ -3613,8 +3622,8 @@ struct WideLds {            // a wave's
   };
 };
 
-// Lists of kPolyMin Gaussians or more a tile on average, on the masks' K, each over kWideBlocks blocks or more on average:
-// a sigma of about 60 elements, as a heavy-tailed field of 407 blocks a Gaussian is half narrow pairs (1280x5120
+// Lists of kPolyMin Gaussians or more a tile on average, on the masks' K, each over kWideBlocks blocks or more on
+// average: a sigma of about 60 elements, as a heavy-tailed field of 407 blocks a Gaussian is half narrow pairs (1280x5120
 // K = 4096, Student-t log-scales: 377 us by moments, 316 by tiles; 32x32 tiles 953 against 827).  A batch, whose
 // layers are mostly of one kind, goes down to 192 (8 fresh layers of 640x640 on 32x32 tiles, by moments and by tiles:
 // 58 and 76 us at 298 blocks, 66 and 92 at 259, 79 and 87 at 226).
@@ -3630,8 +3639,8 @@ __host__ __device__ inline bool wide_field(const Problem& p, int64_t pairs, int6
          q * p.R * p.C >= min_blocks && pairs >= kPolyMin * (int64_t)p.R * p.C && q * pairs >= mean_blocks * p.K;
 }
 
-// The wide Gaussians that a tile's list names again (a bit each marks them once; every time counts): element by element,
-// a Gaussian a lane, over the 2x2 tiles from (tr0, tc0).  No forward makes such lists.
+// The wide Gaussians that a tile's list names again (a bit each marks them once; every time counts): element by
+// element, a Gaussian a lane, over the 2x2 tiles from (tr0, tc0).  No forward makes such lists.
 __device__ __forceinline__ void wide_again(const Problem& p, const float* __restrict__ grad,
                                            const float* __restrict__ row_coords, const float* __restrict__ col_coords,
                                            const GaussEval* __restrict__ ev, const int64_t* __restrict__ tile_ptr,
@@ -3769,71 +3778,72 @@ __device__ __forceinline__ void bwd_wide_body(const Problem& p, const float* __r
   // The n of them, 64 at a time.  A 64's constants are requested before the atomics of the one before: the memory
   // counter is in order, and a load behind atomics would wait for them.
   auto run_list = [&](int32_t n, auto&& id_of) {
-  GaussEval next = zero_eval();
-  int32_t g_next = -1;
-  auto request = [&](int32_t j0) {
-    const int32_t j = lane & (lanes_of(n - j0) - 1);
-    g_next = j0 + j < n ? id_of(j0 + j) : -1;
-    next = zero_eval();
-    if (g_next >= 0) next = load_eval(ev, g_next);
-  };
-  request(0);
-  for (int32_t j0 = 0; j0 < n; j0 += 64) {
-    const int lane = opaque_lane();
-    const int32_t nj = min(64, n - j0), per = lanes_of(nj);
-    const GaussEval my = next;
-    const int32_t g = g_next;
-    float sum[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    bool any = false;
-#pragma unroll 1
-    for (int32_t b0 = 0; b0 < 4; b0 += 64 / per) {
-      const int32_t b = b0 + lane / per;  // the lane's block
-      bool listed = g >= 0 && r0 + 16 * (b >> 1) < p.M && c0 + 16 * (b & 1) < p.N;
-      if (!kQuad && listed) listed = ((bits[b * W + (g >> 5)] >> (g & 31)) & 1u) != 0u;
-      const float4 ba = *reinterpret_cast<const float4*>(&w.block[b][0]), bb = *reinterpret_cast<const float4*>(&w.block[b][4]);
-      const PolyBlock pb{ba.x, ba.y, ba.z, ba.w, bb.x, bb.y, 0, 0};
-      PolyGauss pg = poly_gauss(pb, my);
-      const bool wide = listed && pg.moment && ((fits >> b) & 1u) != 0u;
-      left = left || (listed && !wide);
-      const uint64_t wb = __builtin_amdgcn_ballot_w64(wide);
-      if (wb == 0ull) continue;
-      pg.e0 = poly_e0(pb, my);
-      float mm[6];
-      if (__builtin_amdgcn_ballot_w64(wide && pg.wide) == wb)
-        poly_six<kPolyDeg>(pb, pg, my, w.M[b], mm);
-      else
-        poly_six<kMomentDeg>(pb, pg, my, w.M[b], mm);
-#pragma unroll
-      for (int k = 0; k < 6; ++k) sum[k] += wide ? mm[k] : 0.0f;
-      any = any || wide;
-    }
-    uint64_t taken = __builtin_amdgcn_ballot_w64(any);
-    for (int32_t o = per; o < 64; o <<= 1) {  // the Gaussian's other blocks
-#pragma unroll
-      for (int k = 0; k < 6; ++k) sum[k] += __shfl_xor(sum[k], o, 64);
-      taken |= taken >> o;
-    }
-    if (j0 + 64 < n) request(j0 + 64);
-    // six moments a lane -> eight lanes a Gaussian, half the wave's Gaussians at a time
-    const int32_t to = lane < per && ((taken >> lane) & 1ull) != 0ull ? g : -1;
-    float* ex = w.gt;
-    for (int hf = 0; 32 * hf < nj; ++hf) {
-      if ((lane >> 5) == hf) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) ex[7 * (lane & 31) + k] = sum[k];
-        ex[7 * (lane & 31) + 6] = __int_as_float(to);
+    GaussEval next = zero_eval();
+    int32_t g_next = -1;
+    auto request = [&](int32_t j0) {
+      const int32_t j = lane & (lanes_of(n - j0) - 1);
+      g_next = j0 + j < n ? id_of(j0 + j) : -1;
+      next = zero_eval();
+      if (g_next >= 0) next = load_eval(ev, g_next);
+    };
+    request(0);
+    for (int32_t j0 = 0; j0 < n; j0 += 64) {
+      const int lane = opaque_lane();
+      const int32_t nj = min(64, n - j0), per = lanes_of(nj);
+      const GaussEval my = next;
+      const int32_t g = g_next;
+      float sum[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      bool any = false;
+  #pragma unroll 1
+      for (int32_t b0 = 0; b0 < 4; b0 += 64 / per) {
+        const int32_t b = b0 + lane / per;  // the lane's block
+        bool listed = g >= 0 && r0 + 16 * (b >> 1) < p.M && c0 + 16 * (b & 1) < p.N;
+        if (!kQuad && listed) listed = ((bits[b * W + (g >> 5)] >> (g & 31)) & 1u) != 0u;
+        const float4 ba = *reinterpret_cast<const float4*>(&w.block[b][0]);
+        const float4 bb = *reinterpret_cast<const float4*>(&w.block[b][4]);
+        const PolyBlock pb{ba.x, ba.y, ba.z, ba.w, bb.x, bb.y, 0, 0};
+        PolyGauss pg = poly_gauss(pb, my);
+        const bool wide = listed && pg.moment && ((fits >> b) & 1u) != 0u;
+        left = left || (listed && !wide);
+        const uint64_t wb = __builtin_amdgcn_ballot_w64(wide);
+        if (wb == 0ull) continue;
+        pg.e0 = poly_e0(pb, my);
+        float mm[6];
+        if (__builtin_amdgcn_ballot_w64(wide && pg.wide) == wb)
+          poly_six<kPolyDeg>(pb, pg, my, w.M[b], mm);
+        else
+          poly_six<kMomentDeg>(pb, pg, my, w.M[b], mm);
+  #pragma unroll
+        for (int k = 0; k < 6; ++k) sum[k] += wide ? mm[k] : 0.0f;
+        any = any || wide;
       }
-      wave_sync();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int gi = 8 * i + (lane >> 3), k = lane & 7;
-        const float v = ex[7 * gi + min(k, 5)];
-        const int32_t go = __float_as_int(ex[7 * gi + 6]);
-        if (go >= 0 && k < 6) unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)go + (uint32_t)k), v);
+      uint64_t taken = __builtin_amdgcn_ballot_w64(any);
+      for (int32_t o = per; o < 64; o <<= 1) {  // the Gaussian's other blocks
+  #pragma unroll
+        for (int k = 0; k < 6; ++k) sum[k] += __shfl_xor(sum[k], o, 64);
+        taken |= taken >> o;
       }
-      wave_sync();
+      if (j0 + 64 < n) request(j0 + 64);
+      // six moments a lane -> eight lanes a Gaussian, half the wave's Gaussians at a time
+      const int32_t to = lane < per && ((taken >> lane) & 1ull) != 0ull ? g : -1;
+      float* ex = w.gt;
+      for (int hf = 0; 32 * hf < nj; ++hf) {
+        if ((lane >> 5) == hf) {
+  #pragma unroll
+          for (int k = 0; k < 6; ++k) ex[7 * (lane & 31) + k] = sum[k];
+          ex[7 * (lane & 31) + 6] = __int_as_float(to);
+        }
+        wave_sync();
+  #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int gi = 8 * i + (lane >> 3), k = lane & 7;
+          const float v = ex[7 * gi + min(k, 5)];
+          const int32_t go = __float_as_int(ex[7 * gi + 6]);
+          if (go >= 0 && k < 6) unsafeAtomicAdd(acc_s + (8u * (uint64_t)(uint32_t)go + (uint32_t)k), v);
+        }
+        wave_sync();
+      }
     }
-  }
   };
   if constexpr (kQuad) {
     const int64_t sb = readlane_i64(s, 0), nb = readlane_i64(nl, 0);
@@ -4487,14 +4497,15 @@ __global__ __launch_bounds__(256) void k_selftest_softplus(unsigned long long* o
 // cfg5's reduction at 37-56 us over placements, 32 at 35-39 us (64: the finish cost more than it
 // saved).  Without hot Gaussians the stripes cost the finish 0.5-1.9 us.
 // Few Gaussians on many 16x16 blocks (wide Gaussians: a fresh adapter, or 32x32 tiles, whose four
-// waves add one by one) meet the same lines from every block: S then doubles, up to 32, while there
-// is no more than a slot per block, S * K <= blocks.  A 1280x1280 field of 256 wide Gaussians on 32x32 tiles (61
-// a tile) took its reduction from 100 us with one stripe to 40 with 8 and 35 with 32; a batch of 28
-// such layers from 526 to 366 us; 320x320 with K = 32 from 16.5 to 8.7 us.  With
-// more slots than blocks the finish loses what the reduction gains (28 trained layers of K = 1024:
+// waves add one by one) meet the same lines from every block: S then doubles, up to 32, while that leaves
+// no more than a slot per block, S * K <= blocks (the larger grids' stripes above do not go by K).  A 1280x1280
+// field of 256 wide Gaussians on 32x32 tiles (61 a tile) took its reduction from 100 us with one stripe to 40
+// with 8 and 35 with 32; a batch of 28 such layers from 526 to 366 us; 320x320 with K = 32 from 16.5 to 8.7 us.
+// With more slots than blocks the finish loses what the reduction gains (28 trained layers of K = 1024:
 // 84.6 -> 81.9 us against 5.2 -> 7.5 us at 1.25 slots a block).
-// Above kStripesFewK Gaussians while 2 S * K is: the finish loses sooner what the reduction gains (1280x1280 K = 1024 on
-// 32x32 tiles, trained: reduction 10.2 -> 9.8 us and finish 2.7 -> 3.5 at a slot per block, 10.0 and 3.2 at half of that).
+// Above kStripesFewK Gaussians while 2 S * K is: the finish loses sooner what the reduction gains (1280x1280
+// K = 1024 on 32x32 tiles, trained: reduction 10.2 -> 9.8 us and finish 2.7 -> 3.5 at a slot per block, 10.0 and
+// 3.2 at half of that).
 constexpr int64_t kStripesFewK = 128;
 int32_t backward_stripes(int64_t K, int64_t T, int64_t blocks) {
   int32_t S = T >= 16384 ? 32 : (T >= 8192 ? 8 : (T >= 2048 ? 4 : 1));
@@ -4772,7 +4783,8 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_batch(const uint8_t* __re
 // Layers rendered tile by tile (BatchLayer::pair_render == 0: 32x32 tiles, or 16x16 tiles whose
 // capacity reaches the emission path), over the tile map; the other layers' blocks return.
 template <bool kPoly>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(kPoly ? 7 : 1))) void k_render16_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(kPoly ? 7 : 1))) void k_render16_batch(
+    const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   const uint32_t blk = blockIdx.x;
@@ -4810,7 +4822,8 @@ __global__ __launch_bounds__(kTileThreads) void k_render16x2_batch(const uint8_t
 // Eight waves per SIMD: the batch's dense-tile body fits 64 VGPRs without spilling, and the
 // eighth wave hides more of each tile's load chain (cfg4: 397 -> 383 us).
 template <bool kMaskClamp>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bwd16_batch(const uint8_t* __restrict__ plan, int32_t wide_launched) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bwd16_batch(
+    const uint8_t* __restrict__ plan, int32_t wide_launched) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   int32_t l;
@@ -4820,7 +4833,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
   const BwdLayout L = ly.bl;
   const int64_t T = (int64_t)p.R * p.C;
   const int64_t P = ly.tile_ptr[T];  // pairs beyond the id capacity were never emitted
-  if (wide_launched && ly.wide && wide_field(p, min(P, ly.capacity), kWideBatchMinBlocks, kWideBatchBlocks)) return;  // k_bwd_wide_batch's
+  if (wide_launched && ly.wide && wide_field(p, min(P, ly.capacity), kWideBatchMinBlocks, kWideBatchBlocks))
+    return;  // k_bwd_wide_batch's
   const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
   bwd16_body<int64_t, int64_t, true, kMaskClamp, true, true>(p, grad, ly.row_coords, ly.col_coords, ly.mu, ly.chol_raw,
                                reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
@@ -4829,7 +4843,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8)
 }
 
 // The wide fields of a batch (over the wide map), and what they leave (over the tile map): k_bwd_wide and k_bwd_rest.
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_bwd_wide_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_bwd_wide_batch(
+    const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   int32_t l;
@@ -4844,14 +4859,15 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)
   const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
   const GaussEval* ev = reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval);
   if (p.tile_out == 32)
-    bwd_wide_body<true, false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
-                        lds[wave_id()], bits[wave_id()]);
+    bwd_wide_body<true, false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl,
+                               (int32_t)unit, lds[wave_id()], bits[wave_id()]);
   else
-    bwd_wide_body<false, false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, (int32_t)unit,
-                         lds[wave_id()], bits[wave_id()]);
+    bwd_wide_body<false, false>(p, grad, ly.row_coords, ly.col_coords, ev, ly.tile_ptr, ly.ids, P, ly.bws, ly.bl,
+                                (int32_t)unit, lds[wave_id()], bits[wave_id()]);
 }
 
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_bwd_rest_batch(const uint8_t* __restrict__ plan) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7))) void k_bwd_rest_batch(
+    const uint8_t* __restrict__ plan) {
   const BatchHeader* h = reinterpret_cast<const BatchHeader*>(plan);
   int64_t b0;
   int32_t l;
@@ -4861,8 +4877,9 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(7)
   const int64_t P = min(ly.tile_ptr[(int64_t)p.R * p.C], ly.capacity);
   const float* grad = glob(reinterpret_cast<const float* const*>(plan + h->grad_table_off)[l]);
   bwd16_body<int64_t, int64_t, true, false, true, true, false, true>(
-      p, grad, ly.row_coords, ly.col_coords, ly.mu, ly.chol_raw, reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval),
-      ly.tile_ptr, ly.ids, P, ly.bws, ly.bl, sub_tile(p, (int64_t)blockIdx.x - b0, wave_id()));
+      p, grad, ly.row_coords, ly.col_coords, ly.mu, ly.chol_raw,
+      reinterpret_cast<const GaussEval*>(ly.fws + ly.fl.eval), ly.tile_ptr, ly.ids, P, ly.bws, ly.bl,
+      sub_tile(p, (int64_t)blockIdx.x - b0, wave_id()));
 }
 
 // dL/d(delta) pointers of layers base .. base + count - 1 (count <= kPtrChunk), passed by value.
@@ -5247,8 +5264,8 @@ static int forward_bin(const gf_field_config* cfg, int64_t out_features, int64_t
   } else if (k > 0 && bin_counts_in_lds(p.C, k)) {
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
     const unsigned nbp = (unsigned)((k + kTilesThreads - 1) / kTilesThreads);
-    hipLaunchKernelGGL((k_prep<false, false, 1>), dim3(nbp), dim3(kTilesThreads), 0, st, p, mu, chol_raw, nullptr, ws, L,
-                       num_pairs_dev);
+    hipLaunchKernelGGL((k_prep<false, false, 1>), dim3(nbp), dim3(kTilesThreads), 0, st, p, mu, chol_raw, nullptr, ws,
+                       L, num_pairs_dev);
     GF_LAUNCH_CHECK("k_prep");
     hipLaunchKernelGGL((k_bin_tiles<false, kBinRowsThreads>), dim3((unsigned)p.R), dim3(kBinRowsThreads), 0, st, p,
                        tile_ptr, num_pairs_dev, ws, L, nullptr, nullptr);
@@ -5454,14 +5471,10 @@ static int backward_reduce(const gf_field_config* cfg, int64_t out_features, int
   const int32_t* heavy_list = fws ? reinterpret_cast<const int32_t*>(fws + fwd_layout(p).fill) : nullptr;
   const uint32_t* heavy_count = fws ? &reinterpret_cast<const WsHeader*>(fws)->heavy : nullptr;
   const dim3 grid((unsigned)T);
-  if (tile_ptr_is_int64 && ids_is_int64)
-    launch_bwd<int64_t, int64_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
-  else if (tile_ptr_is_int64)
-    launch_bwd<int64_t, int32_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
-  else if (ids_is_int64)
-    launch_bwd<int32_t, int64_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
-  else
-    launch_bwd<int32_t, int32_t>(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L, heavy_list, heavy_count, counted);
+  auto launch = tile_ptr_is_int64 ? (ids_is_int64 ? launch_bwd<int64_t, int64_t> : launch_bwd<int64_t, int32_t>)
+                                  : (ids_is_int64 ? launch_bwd<int32_t, int64_t> : launch_bwd<int32_t, int32_t>);
+  launch(p, grid, st, grad_delta, row_coords, col_coords, mu, chol_raw, ev, tile_ptr, gaussian_ids, num_pairs, ws, L,
+         heavy_list, heavy_count, counted, nullptr, nullptr);
   GF_LAUNCH_CHECK("k_bwd");
   return GF_OK;
 }
