@@ -3,7 +3,7 @@
 
 A step is one forward (binning + render) and one backward (gradient reduction + chain rule),
 with inputs resident in HBM, issued through the sync-free C ABI path and replayed from a HIP
-graph.  Workloads (BASELINE.json configs):
+graph.  Workloads:
   cfg3 (default, the headline)  one 1280x1280 fp32 delta-W from K=1024 Gaussians
                                 (guass_amd.ops.FieldPlan: three forward launches and the
                                 one-launch backward_direct, which applies the chain rule per
@@ -399,7 +399,7 @@ def model_bench(args) -> int:
         "value": elements / t_batch, "unit": "ΔW elements/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": t_batch * 1e3, "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f32",
-        "data": "synthetic (seeded Gaussian fields, BASELINE.json cfg4 distribution)",
+        "data": "synthetic (seeded Gaussian fields, cfg4 distribution)",
         "config": {"workload": f"cfg4 x{len(probs)} GaussianLinear layers: GaussianFieldBatch.render, every "
                                f"layer's forward on {args.model_tokens} rows, autograd backward (eager)",
                    "layers": len(probs), "sum_out_x_in": int(elements), "k_per_layer": 1024,
@@ -714,7 +714,7 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
-        "data": "synthetic (seeded Gaussian field, BASELINE.json distribution)",
+        "data": "synthetic (seeded Gaussian field, the workload's distribution)",
         "config": {"workload": workload, **shape, "pairs": int(total["pairs"]),
                    "pair_pixel_evals": total["evals"],
                    "binning_state_bytes": int(total["bytes_binning_state"]),

@@ -110,7 +110,7 @@ def make_problem(name: str, M: int, N: int, K: int, log_scale_mean: float, log_s
                         {"seed": seed, "log_scale_mean": log_scale_mean})
 
 
-# BASELINE.json configs.  cfg1..cfg3 and cfg5 are single layers; cfg4 is a list of layers.
+# The benchmark's workloads.  cfg1..cfg3 and cfg5 are single layers; cfg4 is a list of layers.
 def cfg1(seed: int = 0, **kw) -> FieldProblem:
     return make_problem("cfg1_320x320_k64", 320, 320, 64, math.log(4.0), 0.5, seed, **kw)
 

@@ -12,7 +12,7 @@ fixed expected values.  Every file records the torch version it was written with
 Files (numpy .npz, no pickles):
   tiny_ragged.npz   45x70 field, K=12, 16x16 tiles (ragged last tile row and column): inputs,
                     delta, tile_ptr, gaussian ids, d_mu, d_chol_raw, d_amp
-  cfg1_seed0.npz    BASELINE cfg1 (320x320, K=64): inputs except coords (linspace), binning,
+  cfg1_seed0.npz    cfg1 (320x320, K=64): inputs except coords (linspace), binning,
                     gradients, and delta at 2048 fixed positions plus its sum / sum of squares
   softplus.npz      F.softplus of strided views on boundary inputs (bit patterns in and out)
 """

@@ -1,4 +1,4 @@
-"""Parity assertions shared by the GPU tests (bars from BASELINE.json's north star).
+"""Parity assertions shared by the GPU tests (bars of the field path).
 
 * binning (tile_ptr, gaussian ids): bit-exact;
 * delta-W: max |delta - ref| <= 1e-5 * max |ref|  (element-wise relative error is ill-posed

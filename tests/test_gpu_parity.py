@@ -1211,7 +1211,7 @@ def _cfg4_layer(i: int) -> wl.FieldProblem:
 
 
 def test_batch_sd15_layers_against_oracle(device):
-    """One BASELINE cfg4 layer of each of the six SD1.5 attention shapes (320x320, 320x768,
+    """One cfg4 layer of each of the six SD1.5 attention shapes (320x320, 320x768,
     640x640, 640x768, 1280x1280, 1280x768; K = 1024 each) in one batch, against the CPU
     oracle."""
     from guass_amd.ops import FieldBatchPlan
@@ -1360,7 +1360,7 @@ def test_random_fields_sweep(device):
 
 
 def test_cfg4_full_batch_matches_single_fields(device):
-    """BASELINE cfg4 at its workload: all 128 SD1.5 attention layers (K = 1024 each) as one
+    """cfg4 at its workload: all 128 SD1.5 attention layers (K = 1024 each) as one
     FieldBatchPlan, forward and backward, against each layer's own single-field run (the drop-in
     ext path; reference: each adapted layer renders its own delta-W, gaussian_linear.py:162-220).
     Binning is bit-equal for every layer.  delta-W is bit-equal where the single-field render

@@ -7,7 +7,7 @@ libm_f32.h) with g++ and no FP contraction.  These tests pin them bit for bit:
   inputs -- whose checksum the GPU self-test reproduces -- and on samples against
   F.softplus of strided views, which is what the reference CPU path calls;
 * activated Cholesky factor and fp32 covariance (covariance.py:14-38, bounds.py:40-41);
-* tile rectangles (bounds.py:24-75) on the BASELINE configurations.
+* tile rectangles (bounds.py:24-75) on the benchmark's workloads.
 """
 
 from __future__ import annotations

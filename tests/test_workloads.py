@@ -1,4 +1,4 @@
-"""Synthetic workloads: shapes and parameterisation of the BASELINE configurations (CPU)."""
+"""Synthetic workloads: shapes and parameterisation of the benchmark's configurations (CPU)."""
 
 from __future__ import annotations
 
